@@ -260,7 +260,9 @@ int kvc_decode_step(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
 /* Causal chunked prefill.  The n_q query tokens of seq s sit at positions
  * [len_s + pending_s - n_q, len_s + pending_s) (their K/V appended already);
  * row i attends to keys [0, pos_i].  q/gate: bf16 [n_seqs][n_q][Hq][D];
- * out: [n_seqs][n_q][Hq][D]. */
+ * out: [n_seqs][n_q][Hq][D].  A launch too small to fill the GPU splits its
+ * keys over workgroups and folds them through the context's split-K
+ * workspace. */
 int kvc_prefill_attn(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
                      int32_t n_seqs, int32_t n_q, const void* q,
                      const void* gate, void* out, int32_t out_dtype,
@@ -273,7 +275,8 @@ int kvc_prefill_attn(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
  * qkv: [n_seqs][n_q][Hq*2*D + 2*Hkv*D] in kvc_qkv_append's layout, fp32 or
  * bf16 by in_dtype; q_norm, k_norm: device fp32 [D]; out: [n_seqs][n_q][Hq][D]
  * in out_dtype.  Same bits (output and cache) as kvc_qkv_append with q_out and
- * gate_out followed by kvc_prefill_attn on them.  Two launches. */
+ * gate_out followed by kvc_prefill_attn on them.  Two launches, three when the
+ * keys are split (kvc_prefill_attn). */
 int kvc_prefill_step(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
                      int32_t n_seqs, int32_t n_q, const void* qkv,
                      int32_t in_dtype, const void* q_norm, const void* k_norm,

@@ -120,6 +120,17 @@ struct AppendArgs {
     int32_t pos0[kMaxBatch];  // first position written
 };
 
+// prefill work split: a workgroup takes 16 or 32 query rows (ROWS) of one kv
+// head's 4 q heads, one wave per 16 rows of a q head; keys go in tiles of 64.
+// A piece of a split group leaves one fp32 partial per row block: the
+// unnormalised output [ROWS / 4 waves][16 dim groups][64 lanes][4], then
+// (max, sum) per row [ROWS / 4 waves][16 rows][2].  The partials live in the
+// split-K workspace.
+constexpr int kPfKeys = 64;
+constexpr int pf_part_acc(int rows) { return rows / 4 * 16 * 64 * 4; }
+constexpr int pf_part_floats(int rows) { return pf_part_acc(rows) + rows / 4 * 16 * 2; }
+constexpr int64_t pf_max_parts(int rows) { return (int64_t)(kPartBytes / ((size_t)pf_part_floats(rows) * 4)); }
+
 // attention projection row of one token: [Hq][q | gate][D], k [Hkv][D], v [Hkv][D]
 constexpr int kQkvRow = kQHeads * 2 * kHeadDim + 2 * kKvHeads * kHeadDim;
 
@@ -240,9 +251,17 @@ struct PrefillArgs {
     int32_t rope_half;
     int32_t rope_rows;
     int32_t qkv_f32;            // 1: fp32 rows
+    // key split (piece_tiles > 0): a (sequence, kv head) group's keys are cut
+    // into pieces of piece_tiles tiles; a unit is one piece of one group
+    float* part;                // [unit][row block][pf_part_floats(rows)]
+    int32_t rows;               // query rows per workgroup: 16 or 32
+    int32_t piece_tiles;        // 0: no split
+    int32_t n_units;
+    int32_t pb_div;             // parts that a unit's row blocks are dealt to the XCDs in
     int32_t slot[kMaxBatch];
     int32_t q_pos0[kMaxBatch];  // position of query row 0
     int32_t seq_order[kMaxBatch];  // batch indices, most keys first
+    int32_t unit_begin[kMaxBatch + 1];  // first unit of each sequence, in seq_order
 };
 
 // Snapshot copy: per pair, state bytes then the K/V segment.

@@ -321,19 +321,33 @@ __device__ __forceinline__ void merge_waves(const WaveState& st, DecodeSmem& sm,
 __device__ __forceinline__ float sigmoidf_exact(float x) {
     return __builtin_amdgcn_rcpf(1.0f + fast_exp2(-x * 1.4426950408889634f));
 }
-// The output gate sigma(gate) (src/engine.cpp:3563 decode, :2923 prefill):
-// the reference's Schraudolph sigmoid by default, the exact one on request.
-// ref is a kernel argument, uniform over the launch.
-__device__ __forceinline__ float gate_sigmoid(float x, int ref) {
-    return ref ? sigmoid_ref(x) : sigmoidf_exact(x);
-}
-
-// sigmoid(gate) of dims d0 .. d0 + 3 from their bf16 values gw
+// sigmoid(gate) of dims d0 .. d0 + 3 from their bf16 values gw: the output
+// gate sigma(gate) (src/engine.cpp:3563 decode, :2923 prefill), by default the
+// reference's Schraudolph sigmoid (sigmoid_ref's arithmetic and bits), the
+// exact one on request.  gate_ref is a kernel argument, uniform over the
+// launch.  The rare full division (1 + e >= 2^126) is tested once for the four
+// values, in a branch that a wave takes only if one of its lanes needs it:
+// a test and branch per value doubled the epilogues' instructions.
 __device__ __forceinline__ void gate_factors(uint2 gw, int gate_ref, float (&gs)[4]) {
-    gs[0] = gate_sigmoid(bf16lo(gw.x), gate_ref);
-    gs[1] = gate_sigmoid(bf16hi(gw.x), gate_ref);
-    gs[2] = gate_sigmoid(bf16lo(gw.y), gate_ref);
-    gs[3] = gate_sigmoid(bf16hi(gw.y), gate_ref);
+    const float x[4] = {bf16lo(gw.x), bf16hi(gw.x), bf16lo(gw.y), bf16hi(gw.y)};
+    if (gate_ref) {
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            y[i] = 1.0f + schraudolph_exp(-x[i]);
+            const float r = __builtin_amdgcn_rcpf(y[i]);
+            gs[i] = __builtin_fmaf(__builtin_fmaf(-y[i], r, 1.0f), r, r);
+        }
+        const bool big = fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])) >= 0x1p126f;
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(big) != 0, 0)) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (y[i] >= 0x1p126f) gs[i] = 1.0f / y[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) gs[i] = sigmoidf_exact(x[i]);
+    }
 }
 
 // out row = A / L (* gs, the gate factors of dims d0 .. d0 + 3, when
@@ -349,10 +363,8 @@ __device__ __forceinline__ void write_out(void* out, int out_bf16, size_t row_of
         o[3] *= gs[3];
     }
     if (out_bf16) {
-        uint2 w;
-        w.x = pack_bf16x2(o[0], o[1]);
-        w.y = pack_bf16x2(o[2], o[3]);
-        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + row_off + d0) = w;
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + row_off + d0) =
+            make_uint2(cvt_pk_bf16(o[0], o[1]), cvt_pk_bf16(o[2], o[3]));
     } else {
         *reinterpret_cast<float4*>(static_cast<float*>(out) + row_off + d0) =
             make_float4(o[0], o[1], o[2], o[3]);
@@ -1193,8 +1205,6 @@ __global__ __launch_bounds__(kWaves * 64) void decode_kernel(DecodeArgs a) {
 // is 0).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
-constexpr int kPfRows = 32;                 // query positions per workgroup
-constexpr int kPfKeys = 64;                 // keys per tile
 constexpr int kTileElems = kPfKeys * kHeadDim;
 #ifndef KVC_PF_AHEAD
 #define KVC_PF_AHEAD 4
@@ -1202,10 +1212,6 @@ constexpr int kTileElems = kPfKeys * kHeadDim;
 constexpr int kPfAhead = KVC_PF_AHEAD;      // operand fragments read ahead of their MFMAs
 constexpr int kSgMfma = 0x008;              // sched_group_barrier masks: MFMA,
 constexpr int kSgDsRead = 0x100;            //   LDS read
-#ifndef KVC_PF_NT
-#define KVC_PF_NT 1
-#endif
-constexpr int kPfNT = KVC_PF_NT;            // 16-row query tiles per prefill wave (1 or 2)
 
 struct PrefillSmem {  // [buffer][row * 256 + swizzled column]; V first, so V^T reads reach
     uint16_t v[2][kTileElems];   // both buffers with 16-bit immediate offsets from one base
@@ -1269,29 +1275,60 @@ struct PfBuf {
 // RoPE partner of dim d < half is d + half: register ks ^ (half / 32) for
 // half >= 32, lane ^ 16 / ^ 32 for half 8 / 16, the lane's own dims for half
 // 4.  qb receives the bf16 words XOR qflip (the sign of a negative scale).
-template <bool F32IN>
+// The row, the norm weights and (rope_dim 64) the RoPE coefficients are
+// requested first; mid() runs between them and the arithmetic (the first
+// tile's copies, so that they do not wait for it).
+template <bool F32IN, typename Mid>
 __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const float* q_norm,
                                               const float* rope, int rope_rows, int half, int pos, float eps,
-                                              int q4, uint32_t qflip, bf16x8_t (&qb)[8]) {
+                                              int q4, uint32_t qflip, bf16x8_t (&qb)[8], Mid&& mid) {
 #pragma clang fp contract(off)
     float x[8][8];
+    u32x4 raw[8][F32IN ? 2 : 1];
+    float4 wv[8][2];
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
         const size_t e = row + 32 * ks + 8 * q4;
         if constexpr (F32IN) {
             const u32x4* src = reinterpret_cast<const u32x4*>(static_cast<const float*>(qkv) + e);
-            const u32x4 f0 = src[0], f1 = src[1];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                x[ks][j] = __uint_as_float(f0[j]);
-                x[ks][4 + j] = __uint_as_float(f1[j]);
-            }
+            raw[ks][0] = src[0];
+            raw[ks][1] = src[1];
         } else {
-            const u32x4 u = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(qkv) + e);
+            raw[ks][0] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(qkv) + e);
+        }
+    }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                x[ks][2 * j] = bf16lo(u[j]);
-                x[ks][2 * j + 1] = bf16hi(u[j]);
+    for (int ks = 0; ks < 8; ks++) {
+        wv[ks][0] = *reinterpret_cast<const float4*>(q_norm + 32 * ks + 8 * q4);
+        wv[ks][1] = *reinterpret_cast<const float4*>(q_norm + 32 * ks + 8 * q4 + 4);
+    }
+    // RoPE coefficients of dims d0 .. d0 + 7 (d0 = 32 ks + 8 q4 < 2 half):
+    // entries p0 .. p0 + 7 of the position's row (entries 0..3 twice for half 4)
+    auto coef = [&](int d0, float (&c)[8], float (&sn)[8]) {
+        const int p0 = half >= 8 ? (d0 & (half - 1)) : 0;
+        const int o1 = half >= 8 ? 4 : 0;
+        const float* crow = rope + (size_t)pos * half + p0;
+        const float* srow = rope + ((size_t)rope_rows + pos) * half + p0;
+        const float4 c0 = *reinterpret_cast<const float4*>(crow);
+        const float4 c1 = *reinterpret_cast<const float4*>(crow + o1);
+        const float4 s0 = *reinterpret_cast<const float4*>(srow);
+        const float4 s1 = *reinterpret_cast<const float4*>(srow + o1);
+        c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
+        sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
+    };
+    float c32[8] = {}, s32[8] = {};  // half 32: dims 8 q4 and 32 + 8 q4 take the same entries
+    if (half == 32) coef(8 * q4, c32, s32);
+    mid();
+#pragma unroll
+    for (int ks = 0; ks < 8; ks++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (F32IN) {
+                x[ks][j] = __uint_as_float(raw[ks][0][j]);
+                x[ks][4 + j] = __uint_as_float(raw[ks][1][j]);
+            } else {
+                x[ks][2 * j] = bf16lo(raw[ks][0][j]);
+                x[ks][2 * j + 1] = bf16hi(raw[ks][0][j]);
             }
         }
     }
@@ -1311,26 +1348,11 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
     float y[8][8];
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
-        const float4 w0 = *reinterpret_cast<const float4*>(q_norm + 32 * ks + 8 * q4);
-        const float4 w1 = *reinterpret_cast<const float4*>(q_norm + 32 * ks + 8 * q4 + 4);
+        const float4 w0 = wv[ks][0], w1 = wv[ks][1];
         const float w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
         for (int j = 0; j < 8; j++) y[ks][j] = x[ks][j] * rs * w[j];
     }
-    // RoPE coefficients of dims d0 .. d0 + 7 (d0 = 32 ks + 8 q4 < 2 half):
-    // entries p0 .. p0 + 7 of the position's row (entries 0..3 twice for half 4)
-    auto coef = [&](int d0, float (&c)[8], float (&sn)[8]) {
-        const int p0 = half >= 8 ? (d0 & (half - 1)) : 0;
-        const int o1 = half >= 8 ? 4 : 0;
-        const float* crow = rope + (size_t)pos * half + p0;
-        const float* srow = rope + ((size_t)rope_rows + pos) * half + p0;
-        const float4 c0 = *reinterpret_cast<const float4*>(crow);
-        const float4 c1 = *reinterpret_cast<const float4*>(crow + o1);
-        const float4 s0 = *reinterpret_cast<const float4*>(srow);
-        const float4 s1 = *reinterpret_cast<const float4*>(srow + o1);
-        c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w; c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-        sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
-    };
     // half >= 32: registers ks < 2 PM rotate, partner register ks ^ PM
     auto rotate_regs = [&](auto pmc) {
         constexpr int PM = decltype(pmc)::value;
@@ -1338,10 +1360,15 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
 #pragma unroll
         for (int ks = 0; ks < 2 * PM; ks++) {
             float c[8], sn[8];
-            coef(32 * ks + 8 * q4, c, sn);
+            if constexpr (PM > 1) coef(32 * ks + 8 * q4, c, sn);
 #pragma unroll
-            for (int j = 0; j < 8; j++)
+            for (int j = 0; j < 8; j++) {
+                if constexpr (PM == 1) {
+                    c[j] = c32[j];
+                    sn[j] = s32[j];
+                }
                 z[ks][j] = ks < PM ? y[ks][j] * c[j] - y[ks ^ PM][j] * sn[j] : y[ks][j] * c[j] + y[ks ^ PM][j] * sn[j];
+            }
         }
 #pragma unroll
         for (int ks = 0; ks < 2 * PM; ks++)
@@ -1387,9 +1414,12 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
     }
 }
 
-// NT = 16-row query tiles per wave: NT = 2 runs 4 waves (one per q head of
-// the group, 32 rows each); NT = 1 runs 8 waves (q head, row half), two per
-// SIMD, so one wave's MFMAs overlap the other's LDS reads and softmax.
+// A wave takes one q head of the group and 16 query rows, so a workgroup of
+// ROWS = 32 rows has 8 waves, two per SIMD: one wave's MFMAs overlap the
+// other's LDS reads and softmax, and each K/V tile serves 32 rows.  ROWS = 16
+// (4 waves, one per SIMD) is for launches that leave CUs idle anyway: half the
+// rows per workgroup halves its q arithmetic, softmax and gate epilogue, which
+// share the SIMDs' VALUs (prefill_rows in the host code has the rule).
 //
 // The per-tile VALU work is kept small:
 //  - tiles are fetched with the scalar-base form of the LDS DMA, with
@@ -1411,37 +1441,59 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
 // from the rows in the epilogue (fp32 rounded to bf16 first, as the producer
 // writes it), so the result has the bits of kvc_qkv_append + the plain
 // kernel.
-template <int NT, int PROD>
-__global__ __launch_bounds__(64 * 8 / NT) __attribute__((amdgpu_waves_per_eu(2 / NT, 2 / NT)))
+//
+// SPLIT: a workgroup takes one piece (a.piece_tiles tiles) of its query
+// block's keys and leaves its unnormalised output and row statistics in the
+// workspace for prefill_combine_kernel; a block that one piece covers is
+// finished here.  Chosen by the host for launches that would leave most CUs
+// idle (prefill_piece_tiles).
+template <int ROWS, int PROD, bool SPLIT>
+__global__ __launch_bounds__(ROWS * 16) __attribute__((amdgpu_waves_per_eu(ROWS / 16, ROWS / 16)))
 void prefill_mfma_kernel(PrefillArgs a) {
     constexpr bool PRODUCE = PROD != 0;
     constexpr bool F32IN = PROD == 2;
-    constexpr int kWavesPf = 8 / NT;
-    constexpr int kRowsPerWave = 16 * NT;
+    constexpr int kWavesPf = ROWS / 4;
     constexpr int kLoadRows = kPfKeys / kWavesPf;  // tile rows each wave loads
     __shared__ PrefillSmem sm;
     // Workgroup b runs on XCD b % 8.  The n_pb query blocks of one (sequence,
     // kv head) group share its K/V, so they go to one XCD (one L2), in
     // consecutive dispatch rounds; groups are taken most keys first (the
     // sequence order is sorted on the host) and, inside a group, the later
-    // (longer) query blocks first.
-    const int n_pb = (a.n_q + kPfRows - 1) / kPfRows;
+    // (longer) query blocks first.  Split launches do the same with (group,
+    // piece) units: the query blocks of a unit read the same keys.  When the
+    // units do not divide evenly over the XCDs, each is dealt out as a.pb_div
+    // interleaved parts (one sequence alone has 4 groups, half the XCDs).
+    const int n_pb = (a.n_q + ROWS - 1) / ROWS;
+    const int per_part = (n_pb + a.pb_div - 1) / a.pb_div;
     const int xcd = blockIdx.x & 7, round = blockIdx.x >> 3;
-    const int grp = (round / n_pb) * 8 + xcd;
-    if (grp >= a.n_groups) return;
-    const int pb = n_pb - 1 - round % n_pb;
+    const int dealt = (round / per_part) * 8 + xcd;
+    const int unit = dealt / a.pb_div;
+    if (unit >= (SPLIT ? a.n_units : a.n_groups)) return;
+    const int pb = n_pb - 1 - (round % per_part * a.pb_div + dealt % a.pb_div);
+    if (pb < 0) return;
+    int grp = unit, piece = 0;
+    if constexpr (SPLIT) {
+        int so = 0;
+        while (unit >= a.unit_begin[so + 1]) so++;
+        const int v = unit - a.unit_begin[so];
+        grp = so * kKvHeads + v % kKvHeads;
+        piece = v / kKvHeads;
+    }
     const int h = grp % kKvHeads;
     const int s = a.seq_order[grp / kKvHeads];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (LDS DMA base)
     const int q4 = lane >> 4, r16 = lane & 15;
     const int g = wave & 3;            // q head of the group
-    const int rw0 = (wave >> 2) * kRowsPerWave;  // first row of the wave within the tile
+    const int rw0 = (wave >> 2) * 16;  // first row of the wave within the tile
     const int pos0 = a.q_pos0[s];
-    const int row0 = pb * kPfRows;                     // first query row of the tile
-    const int rows = min(kPfRows, a.n_q - row0);
+    const int row0 = pb * ROWS;                     // first query row of the tile
+    const int rows = min(ROWS, a.n_q - row0);
     const int kmax = pos0 + row0 + rows;               // keys [0, kmax) are visible
     const int n_tiles = (kmax + kPfKeys - 1) / kPfKeys;
+    const int t_begin = SPLIT ? piece * a.piece_tiles : 0;
+    if (SPLIT && t_begin >= n_tiles) return;
+    const int t_end = SPLIT ? min(t_begin + a.piece_tiles, n_tiles) : n_tiles;
     const int n_blocks = (kmax + kBlockTok - 1) / kBlockTok;
     const int32_t* trow = a.table + (size_t)a.slot[s] * a.table_stride;
     constexpr size_t kUnitElems = (size_t)kBlockTok * kHeadDim;
@@ -1452,32 +1504,9 @@ void prefill_mfma_kernel(PrefillArgs a) {
     // and are read with v_readlane: no dependent table load on the fetch
     // path.  The first window's are requested before Q, so the wait for them
     // (the load counter completes in order) does not also wait for Q.
-    int idw0 = 0;
-    int idv = lane < n_blocks ? trow[lane] : 0;
+    int idw0 = 2 * t_begin;
+    int idv = idw0 + lane < n_blocks ? trow[idw0 + lane] : 0;
     __builtin_amdgcn_sched_barrier(0);
-
-    // Q^T as the B operand: qb[nt][ks] = q[row rw0 + 16nt + r16][d 32ks + 8q4 .. +7]
-    bf16x8_t qb[NT][8];
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const int r = row0 + min(rw0 + 16 * nt + r16, rows - 1);
-        if constexpr (PRODUCE) {
-            const size_t row = ((size_t)s * a.n_q + r) * kQkvRow + (size_t)(h * kGroup + g) * 2 * kHeadDim;
-            prefill_q_row<F32IN>(a.qkv, row, a.q_norm, a.rope, a.rope_rows, a.rope_half, pos0 + r, a.eps, q4, qflip,
-                                 qb[nt]);
-        } else {
-            const uint16_t* qr = a.q + (((size_t)s * a.n_q + r) * kQHeads + h * kGroup + g) * kHeadDim;
-#pragma unroll
-            for (int ks = 0; ks < 8; ks++) {
-                u32x4 x = *reinterpret_cast<const u32x4*>(qr + 32 * ks + 8 * q4);
-                x[0] ^= qflip;
-                x[1] ^= qflip;
-                x[2] ^= qflip;
-                x[3] ^= qflip;
-                qb[nt][ks] = as_bf16x8(x);
-            }
-        }
-    }
 
     // wave w loads tile rows kLoadRows*w .., two per instruction (lanes 0-31:
     // row r0, lanes 32-63: the next row); lane l fills chunk position l % 32
@@ -1513,19 +1542,38 @@ void prefill_mfma_kernel(PrefillArgs a) {
     auto issue_k = [&](int t, int buf) { issue_rows(a.kpool, cbk, 5, lds_addr(&sm.k[buf][0]), t); };
     auto issue_v = [&](int t, int buf) { issue_rows(a.vpool, cbv, 6, lds_addr(&sm.v[buf][0]), t); };
 
-    // With NT = 2 the accumulators outgrow the VGPRs: an (empty) statement
-    // with an AGPR operand makes the compiler select the AGPR-accumulator form
-    // of the MFMAs, so O^T lives in AGPRs.
-    if constexpr (NT == 2) asm volatile("" ::"a"(0));
-    f32x4 o[16][NT], ol[NT];  // ol: the all-ones row block (softmax denominator)
-    float m_run[NT];
+    // Q^T as the B operand: qb[ks] = q[row rw0 + r16][d 32ks + 8q4 .. +7]
+    // The first tile's copies are issued right after the q loads and before the
+    // q arithmetic of the prefill step.
+    auto issue_first = [&] {
+        issue_k(t_begin, 0);
+        issue_v(t_begin, 0);
+    };
+    bf16x8_t qb[8];
+    const int r = row0 + min(rw0 + r16, rows - 1);
+    if constexpr (PRODUCE) {
+        const size_t row = ((size_t)s * a.n_q + r) * kQkvRow + (size_t)(h * kGroup + g) * 2 * kHeadDim;
+        prefill_q_row<F32IN>(a.qkv, row, a.q_norm, a.rope, a.rope_rows, a.rope_half, pos0 + r, a.eps, q4, qflip,
+                             qb, issue_first);
+    } else {
+        const uint16_t* qr = a.q + (((size_t)s * a.n_q + r) * kQHeads + h * kGroup + g) * kHeadDim;
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-#pragma unroll
-        for (int dt = 0; dt < 16; dt++) o[dt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        ol[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        m_run[nt] = kNegBig;
+        for (int ks = 0; ks < 8; ks++) {
+            u32x4 x = *reinterpret_cast<const u32x4*>(qr + 32 * ks + 8 * q4);
+            x[0] ^= qflip;
+            x[1] ^= qflip;
+            x[2] ^= qflip;
+            x[3] ^= qflip;
+            qb[ks] = as_bf16x8(x);
+        }
     }
+    if constexpr (!PRODUCE) issue_first();
+
+    f32x4 o[16], ol;  // ol: the all-ones row block (softmax denominator)
+    float m_run = kNegBig;
+#pragma unroll
+    for (int dt = 0; dt < 16; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    ol = f32x4{0.f, 0.f, 0.f, 0.f};
     const bf16x8_t ones = as_bf16x8(u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
 
     // Per-lane LDS byte addresses of the operand fragments in buffer 0 (the
@@ -1544,11 +1592,11 @@ void prefill_mfma_kernel(PrefillArgs a) {
             vaddr[dt] = v0 + w * 512 + 16 * (2 * (dt ^ w) + ((r16 & 3) >> 1)) + 8 * (r16 & 1);
     }
 
-    // S^T tiles: s[kt][nt], lane holds keys 16kt + 4q4 + i of row 16nt + r16.
+    // S^T tiles: s[kt], lane holds keys 16kt + 4q4 + i of row r16.
     // Steps i = (ks, kt) run d-slice outer, key subtile inner, so consecutive
     // MFMAs feed different accumulators; the 32 K fragments are read kPfAhead
     // steps ahead of their MFMAs through a register ring.
-    auto compute_s = [&](auto bufc, f32x4 (&s)[4][NT]) {
+    auto compute_s = [&](auto bufc, f32x4 (&s)[4]) {
         constexpr uint32_t kOff = decltype(bufc)::value * (uint32_t)sizeof(sm.k[0]);
         bf16x8_t kf[kPfAhead];
         auto read_kfrag = [&](int i) {
@@ -1562,9 +1610,7 @@ void prefill_mfma_kernel(PrefillArgs a) {
             const int ks = i >> 2, kt = i & 3;
             const bf16x8_t ka = kf[i % kPfAhead];
             if (i + kPfAhead < 32) read_kfrag(i + kPfAhead);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-                s[kt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[nt][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[kt][nt], 0, 0, 0);
+                s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[kt], 0, 0, 0);
         }
     };
 
@@ -1583,7 +1629,7 @@ void prefill_mfma_kernel(PrefillArgs a) {
         for (int dt = 0; dt < 16; dt++) asm volatile("" : "+v"(vaddr[dt]));
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        if (t + 1 < n_tiles) {
+        if (t + 1 < t_end) {
             if (2 * (t + 1) + 1 - idw0 >= 64 && 2 * (t + 1) < n_blocks) {  // uniform: next id window
                 idw0 = 2 * (t + 1);
                 idv = idw0 + lane < n_blocks ? trow[idw0 + lane] : 0;
@@ -1591,18 +1637,18 @@ void prefill_mfma_kernel(PrefillArgs a) {
             issue_k(t + 1, B ^ 1);
             issue_v(t + 1, B ^ 1);
         }
-        f32x4 st[4][NT];
+        f32x4 st[4];
         // the MFMA runs (S here, P.V below) issue at raised wave priority, so
         // on a SIMD the wave feeding the matrix pipe goes ahead of the other
         // wave's softmax VALU work
         __builtin_amdgcn_s_setprio(1);
         compute_s(PfBuf<B>{}, st);
-        // pin the pipeline: kPfAhead reads, then (1 read, NT MFMAs) per step
+        // pin the pipeline: kPfAhead reads, then (1 read, 1 MFMA) per step
         __builtin_amdgcn_sched_group_barrier(kSgDsRead, kPfAhead, 0);
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             if (i + kPfAhead < 32) __builtin_amdgcn_sched_group_barrier(kSgDsRead, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(kSgMfma, NT, 0);
+            __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
         }
         __builtin_amdgcn_s_setprio(0);
 
@@ -1615,65 +1661,53 @@ void prefill_mfma_kernel(PrefillArgs a) {
         const bool full = t * kPfKeys + kPfKeys - 1 <= pos0 + row0 + rw0 && t * kPfKeys + kPfKeys <= kmax;
         if (!full) {
             asm volatile("");
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const int qpos = pos0 + row0 + rw0 + 16 * nt + r16;
-#pragma unroll
-                for (int kt = 0; kt < 4; kt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int kp = t * kPfKeys + 16 * kt + 4 * q4 + i;
-                        st[kt][nt][i] = (kp <= qpos && kp < kmax) ? st[kt][nt][i] * c : kNegBig;
-                    }
-            }
-        }
-        const float cs = full ? c : 1.f;
-        bool need = false;
-        float mt[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            float mx = kNegBig;
+            const int qpos = pos0 + row0 + rw0 + r16;
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[kt][nt][i]);
-            mx = max_xor16(mx);
-            mx = max_xor32(mx);
-            mt[nt] = full ? mx * c : mx;
-            need |= mt[nt] > m_run[nt] + kRescaleSlack;
+                for (int i = 0; i < 4; i++) {
+                    const int kp = t * kPfKeys + 16 * kt + 4 * q4 + i;
+                    st[kt][i] = (kp <= qpos && kp < kmax) ? st[kt][i] * c : kNegBig;
+                }
         }
+        const float cs = full ? c : 1.f;
+        bool need = false;
+        float mt;
+        float mx = kNegBig;
+#pragma unroll
+        for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[kt][i]);
+        mx = max_xor16(mx);
+        mx = max_xor32(mx);
+        mt = full ? mx * c : mx;
+        need |= mt > m_run + kRescaleSlack;
         if (__builtin_amdgcn_ballot_w64(need) != 0) {  // uniform; rows that keep their max scale by 1
+            const bool up = mt > m_run + kRescaleSlack;
+            const float cr = up ? fast_exp2(m_run - mt) : 1.f;
+            m_run = up ? mt : m_run;
+            // the scaled values re-enter the accumulators through an MFMA
+            // with zero operands, which keeps them in the MFMA register class
+            const bf16x8_t z8 = {};
 #pragma unroll
-            for (int nt = 0; nt < NT; nt++) {
-                const bool up = mt[nt] > m_run[nt] + kRescaleSlack;
-                const float cr = up ? fast_exp2(m_run[nt] - mt[nt]) : 1.f;
-                m_run[nt] = up ? mt[nt] : m_run[nt];
-                // the scaled values re-enter the accumulators through an MFMA
-                // with zero operands, which keeps them in the MFMA register class
-                const bf16x8_t z8 = {};
-#pragma unroll
-                for (int dt = 0; dt < 16; dt++)
-                    o[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z8, z8, o[dt][nt] * cr, 0, 0, 0);
-                ol[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z8, z8, ol[nt] * cr, 0, 0, 0);
-            }
+            for (int dt = 0; dt < 16; dt++)
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z8, z8, o[dt] * cr, 0, 0, 0);
+            ol = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z8, z8, ol * cr, 0, 0, 0);
         }
         // P^T as the B operand (bf16), k-slot order (4q4 + i, 16 + 4q4 + i);
         // p = 2^(s * cs - m) with one rounding before the exponential
-        bf16x8_t pb_[NT][2];
+        bf16x8_t pb_[2];
+        const float nm = -m_run;
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++) {
-            const float nm = -m_run[nt];
+        for (int kk = 0; kk < 2; kk++) {
+            u32x4 w;
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                u32x4 w;
-#pragma unroll
-                for (int hf = 0; hf < 2; hf++) {
-                    const f32x4 sv = st[2 * kk + hf][nt];
-                    w[2 * hf] = cvt_pk_bf16(fast_exp2(fmaf(sv[0], cs, nm)), fast_exp2(fmaf(sv[1], cs, nm)));
-                    w[2 * hf + 1] = cvt_pk_bf16(fast_exp2(fmaf(sv[2], cs, nm)), fast_exp2(fmaf(sv[3], cs, nm)));
-                }
-                pb_[nt][kk] = as_bf16x8(w);
+            for (int hf = 0; hf < 2; hf++) {
+                const f32x4 sv = st[2 * kk + hf];
+                w[2 * hf] = cvt_pk_bf16(fast_exp2(fmaf(sv[0], cs, nm)), fast_exp2(fmaf(sv[1], cs, nm)));
+                w[2 * hf + 1] = cvt_pk_bf16(fast_exp2(fmaf(sv[2], cs, nm)), fast_exp2(fmaf(sv[3], cs, nm)));
             }
+            pb_[kk] = as_bf16x8(w);
         }
 
         // O^T += V^T . P^T; the V^T operand of lane (q4, r16) is V[keys
@@ -1700,73 +1734,151 @@ void prefill_mfma_kernel(PrefillArgs a) {
             const int kk = i >> 4, dt = i & 15;
             const bf16x8_t va = vf[i % kPfAhead];
             if (i + kPfAhead < 32) read_vfrag(i + kPfAhead);
-#pragma unroll
-            for (int nt = 0; nt < NT; nt++)
-                o[dt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb_[nt][kk], o[dt][nt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb_[kk], o[dt], 0, 0, 0);
         }
 #pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
             for (int kk = 0; kk < 2; kk++)
-                ol[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb_[nt][kk], ol[nt], 0, 0, 0);
+                ol = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb_[kk], ol, 0, 0, 0);
         __builtin_amdgcn_sched_group_barrier(kSgDsRead, 2 * kPfAhead, 1);
 #pragma unroll
         for (int i = 0; i < 32; i++) {
             if (i + kPfAhead < 32) __builtin_amdgcn_sched_group_barrier(kSgDsRead, 2, 1);
-            __builtin_amdgcn_sched_group_barrier(kSgMfma, NT, 1);
+            __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 1);
         }
         __builtin_amdgcn_s_setprio(0);
     };
 
-    issue_k(0, 0);
-    issue_v(0, 0);
-    for (int t = 0; t < n_tiles; t += 2) {
+    for (int t = t_begin; t < t_end; t += 2) {
         step(PfBuf<0>{}, t);
-        if (t + 1 < n_tiles) step(PfBuf<1>{}, t + 1);
+        if (t + 1 < t_end) step(PfBuf<1>{}, t + 1);
+    }
+    if constexpr (SPLIT) {
+        if (n_tiles > a.piece_tiles) {
+            // 1-KiB stores: lane (q4, r16) holds dims 16dt + 4q4 .. +3 of row
+            // r16.  A row that sees no key of the piece leaves m = kNegBig,
+            // which weighs 0 against the piece holding key 0.
+            if (rw0 < rows) {
+                float* part = a.part + ((size_t)unit * n_pb + pb) * pf_part_floats(ROWS);
+                float* acc = part + (size_t)wave * 16 * 64 * 4 + lane * 4;
+#pragma unroll
+                for (int dt = 0; dt < 16; dt++) *reinterpret_cast<f32x4*>(acc + dt * 256) = o[dt];
+                if (lane < 16)
+                    *reinterpret_cast<float2*>(part + pf_part_acc(ROWS) + (wave * 16 + r16) * 2) =
+                        make_float2(m_run, ol[0]);
+            }
+            return;
+        }
     }
     // epilogue: every row of a lane's ol block holds its query row's
-    // denominator; normalise, gate, store
+    // denominator; normalise, gate, store.  The 64 values a lane finishes are
+    // VALU work that the CU's waves share (about 5 us per 32-row workgroup
+    // before, 2.5 of them the gate's per-value division test and the software
+    // rounding), so both take their short forms here; the gate words are all
+    // requested before the first store, which a load cannot pass.  With the
+    // first tile's copies issued ahead of the q arithmetic: 64 sequences of
+    // 128 rows over 256-3072 keys, 363 -> 341 us per layer.
+    const float l = ol[0];
+    const int rl = rw0 + r16;
+    if (rl >= rows) return;
+    const size_t orow = (((size_t)s * a.n_q + row0 + rl) * kQHeads + h * kGroup + g) * kHeadDim;
+    const bool gated = PRODUCE || a.gate;
+    uint2 gw[16];
+    if (gated) {
+        [[maybe_unused]] const size_t ge =
+            ((size_t)s * a.n_q + row0 + rl) * kQkvRow + (size_t)(h * kGroup + g) * 2 * kHeadDim + kHeadDim;
+        if constexpr (F32IN) {
+            float4 f[16];
 #pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-        const float l = ol[nt][0];
-        const int rl = rw0 + 16 * nt + r16;
-        if (rl >= rows) continue;
-        const size_t orow = (((size_t)s * a.n_q + row0 + rl) * kQHeads + h * kGroup + g) * kHeadDim;
-        const float inv = __builtin_amdgcn_rcpf(l);
+            for (int dt = 0; dt < 16; dt++)
+                f[dt] = *reinterpret_cast<const float4*>(static_cast<const float*>(a.qkv) + ge + 16 * dt + 4 * q4);
 #pragma unroll
-        for (int dt = 0; dt < 16; dt++) {
-            const int d0 = 16 * dt + 4 * q4;
-            float v4[4] = {o[dt][nt][0] * inv, o[dt][nt][1] * inv, o[dt][nt][2] * inv, o[dt][nt][3] * inv};
-            if (PRODUCE || a.gate) {
-                uint2 gw;
-                if constexpr (PRODUCE) {
-                    const size_t ge = ((size_t)s * a.n_q + row0 + rl) * kQkvRow +
-                                      (size_t)(h * kGroup + g) * 2 * kHeadDim + kHeadDim + d0;
-                    if constexpr (F32IN) {
-                        const float4 f = *reinterpret_cast<const float4*>(static_cast<const float*>(a.qkv) + ge);
-                        gw = make_uint2(cvt_pk_bf16(f.x, f.y), cvt_pk_bf16(f.z, f.w));
-                    } else {
-                        gw = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a.qkv) + ge);
-                    }
-                } else {
-                    gw = *reinterpret_cast<const uint2*>(a.gate + orow + d0);
-                }
-                v4[0] *= gate_sigmoid(bf16lo(gw.x), a.gate_ref);
-                v4[1] *= gate_sigmoid(bf16hi(gw.x), a.gate_ref);
-                v4[2] *= gate_sigmoid(bf16lo(gw.y), a.gate_ref);
-                v4[3] *= gate_sigmoid(bf16hi(gw.y), a.gate_ref);
-            }
-            if (a.out_bf16) {
-                uint2 w;
-                w.x = pack_bf16x2(v4[0], v4[1]);
-                w.y = pack_bf16x2(v4[2], v4[3]);
-                *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + orow + d0) = w;
-            } else {
-                *reinterpret_cast<float4*>(static_cast<float*>(a.out) + orow + d0) =
-                    make_float4(v4[0], v4[1], v4[2], v4[3]);
+            for (int dt = 0; dt < 16; dt++)
+                gw[dt] = make_uint2(cvt_pk_bf16(f[dt].x, f[dt].y), cvt_pk_bf16(f[dt].z, f[dt].w));
+        } else {
+            const uint16_t* grow = PRODUCE ? static_cast<const uint16_t*>(a.qkv) + ge : a.gate + orow;
+#pragma unroll
+            for (int dt = 0; dt < 16; dt++) gw[dt] = *reinterpret_cast<const uint2*>(grow + 16 * dt + 4 * q4);
+        }
+    }
+#pragma unroll
+    for (int dt = 0; dt < 16; dt++) {
+        float gs[4] = {1.f, 1.f, 1.f, 1.f};
+        if (gated) gate_factors(gw[dt], a.gate_ref, gs);
+        const float A[4] = {o[dt][0], o[dt][1], o[dt][2], o[dt][3]};
+        write_out(a.out, a.out_bf16, orow, 16 * dt + 4 * q4, gated, gs, l, A);
+    }
+}
+
+// Folds the pieces of a split prefill: out = sum(w_p acc_p) / sum(w_p l_p),
+// w_p = 2^(m_p - max m), gated and stored.  A wave takes one 16-row, 16-dim
+// group of a (sequence, kv head, query block, q head) in the layout that the
+// pieces stored it in (1 KiB per piece and load), so a 32-row block of one
+// sequence is folded by 512 waves.
+constexpr int kPfFold = 16;  // pieces requested at once
+template <int ROWS>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
+    const int n_pb = (a.n_q + ROWS - 1) / ROWS;
+    const int lane = threadIdx.x & 63, q4 = lane >> 4, r16 = lane & 15;
+    const int dt = (blockIdx.x & 3) * 4 + (threadIdx.x >> 6);
+    const int wave = (blockIdx.x >> 2) % (ROWS / 4);  // of the prefill workgroup: q head, 16-row group
+    const int blk = blockIdx.x / ROWS;
+    const int pb = blk % n_pb, grp = blk / n_pb;
+    const int h = grp % kKvHeads, so = grp / kKvHeads, s = a.seq_order[so];
+    const int row0 = pb * ROWS, rows = min(ROWS, a.n_q - row0);
+    const int rl = (wave >> 2) * 16 + r16;
+    const int n_tiles = (a.q_pos0[s] + row0 + rows + kPfKeys - 1) / kPfKeys;
+    const int np = (n_tiles + a.piece_tiles - 1) / a.piece_tiles;
+    if (np <= 1 || (wave >> 2) * 16 >= rows) return;
+    const int head = h * kGroup + (wave & 3), d0 = 16 * dt + 4 * q4;
+    const size_t row = (size_t)s * a.n_q + row0 + min(rl, rows - 1);
+    const size_t o = (row * kQHeads + head) * kHeadDim;
+    const bool gated = a.qkv || a.gate;
+    uint2 gw = make_uint2(0u, 0u);
+    float4 gf = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (gated) {  // requested ahead of the partials
+        const size_t ge = row * kQkvRow + (size_t)head * 2 * kHeadDim + kHeadDim + d0;
+        if (a.qkv && a.qkv_f32)
+            gf = *reinterpret_cast<const float4*>(static_cast<const float*>(a.qkv) + ge);
+        else
+            gw = *reinterpret_cast<const uint2*>(a.qkv ? static_cast<const uint16_t*>(a.qkv) + ge : a.gate + o + d0);
+    }
+    const size_t step = (size_t)kKvHeads * n_pb * pf_part_floats(ROWS);  // between pieces
+    const float* part = a.part + ((size_t)(a.unit_begin[so] + h) * n_pb + pb) * pf_part_floats(ROWS);
+    const float* acc = part + ((size_t)wave * 16 + dt) * 256 + lane * 4;
+    const float* ml = part + pf_part_acc(ROWS) + (wave * 16 + r16) * 2;
+    float A[4] = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f, m = kNegBig;
+    for (int p0 = 0; p0 < np; p0 += kPfFold) {
+        f32x4 x[kPfFold];
+        float2 st[kPfFold];
+#pragma unroll
+        for (int j = 0; j < kPfFold; j++) {  // past the end: the last piece again, weight 0
+            const size_t off = (size_t)min(p0 + j, np - 1) * step;
+            st[j] = *reinterpret_cast<const float2*>(ml + off);
+            x[j] = *reinterpret_cast<const f32x4*>(acc + off);
+        }
+        float mx = m;
+#pragma unroll
+        for (int j = 0; j < kPfFold; j++) mx = fmaxf(mx, st[j].x);
+        const float cr = fast_exp2(m - mx);
+        m = mx;
+        l *= cr;
+#pragma unroll
+        for (int i = 0; i < 4; i++) A[i] *= cr;
+#pragma unroll
+        for (int j = 0; j < kPfFold; j++) {
+            if (p0 + j < np) {
+                const float w = fast_exp2(st[j].x - m);
+                l = fmaf(w, st[j].y, l);
+#pragma unroll
+                for (int i = 0; i < 4; i++) A[i] = fmaf(w, x[j][i], A[i]);
             }
         }
     }
+    if (a.qkv && a.qkv_f32) gw = make_uint2(cvt_pk_bf16(gf.x, gf.y), cvt_pk_bf16(gf.z, gf.w));
+    float gs[4] = {1.f, 1.f, 1.f, 1.f};
+    if (gated) gate_factors(gw, a.gate_ref, gs);
+    if (rl < rows) write_out(a.out, a.out_bf16, o, d0, gated, gs, l, A);
 }
 
 // ---------------------------------------------------------------------------
@@ -3479,15 +3591,25 @@ int launch_checksum(const ChecksumArgs& a, void* stream) {
     return (int)hipGetLastError();
 }
 
-int launch_prefill(const PrefillArgs& a, void* stream) {
-    const int grid = 8 * ((a.n_groups + 7) / 8) * ((a.n_q + kPfRows - 1) / kPfRows);
-    const hipStream_t st = (hipStream_t)stream;
+template <int ROWS, bool SPLIT>
+static void launch_prefill_t(const PrefillArgs& a, hipStream_t st) {
+    const int n = SPLIT ? a.n_units : a.n_groups, n_pb = (a.n_q + ROWS - 1) / ROWS;
+    const int grid = 8 * ((n * a.pb_div + 7) / 8) * ((n_pb + a.pb_div - 1) / a.pb_div);
     if (a.qkv && a.qkv_f32)
-        hipLaunchKernelGGL((prefill_mfma_kernel<kPfNT, 2>), dim3(grid), dim3(64 * 8 / kPfNT), 0, st, a);
+        hipLaunchKernelGGL((prefill_mfma_kernel<ROWS, 2, SPLIT>), dim3(grid), dim3(ROWS * 16), 0, st, a);
     else if (a.qkv)
-        hipLaunchKernelGGL((prefill_mfma_kernel<kPfNT, 1>), dim3(grid), dim3(64 * 8 / kPfNT), 0, st, a);
+        hipLaunchKernelGGL((prefill_mfma_kernel<ROWS, 1, SPLIT>), dim3(grid), dim3(ROWS * 16), 0, st, a);
     else
-        hipLaunchKernelGGL((prefill_mfma_kernel<kPfNT, 0>), dim3(grid), dim3(64 * 8 / kPfNT), 0, st, a);
+        hipLaunchKernelGGL((prefill_mfma_kernel<ROWS, 0, SPLIT>), dim3(grid), dim3(ROWS * 16), 0, st, a);
+    if (SPLIT) hipLaunchKernelGGL(prefill_combine_kernel<ROWS>, dim3(a.n_groups * n_pb * ROWS), dim3(256), 0, st, a);
+}
+
+int launch_prefill(const PrefillArgs& a, void* stream) {
+    const hipStream_t st = (hipStream_t)stream;
+    if (a.rows == 16)
+        a.piece_tiles > 0 ? launch_prefill_t<16, true>(a, st) : launch_prefill_t<16, false>(a, st);
+    else
+        a.piece_tiles > 0 ? launch_prefill_t<32, true>(a, st) : launch_prefill_t<32, false>(a, st);
     return (int)hipGetLastError();
 }
 
