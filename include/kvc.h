@@ -327,7 +327,8 @@ int kvc_state_ptrs(kvc_ctx* ctx, int32_t seq, int32_t ssm_layer, void** rec,
  * (each within 2 ulp of the exact function) instead.  Built for
  * 32 v-heads, 16 k-heads, 128 x 128 heads, a 3-row window and 8192 channels
  * (KVC_ERR_UNSUPPORTED otherwise); one seq's n_tok rows of proj must span
- * less than 2 GiB (KVC_ERR_RANGE otherwise). */
+ * less than 2 GiB (KVC_ERR_RANGE otherwise).  Calls of few sequences and many
+ * tokens run as several launches through the context's split-K workspace. */
 int kvc_deltanet_step(kvc_ctx* ctx, int32_t ssm_layer, const int32_t* seqs,
                       int32_t n_seqs, int32_t n_tok, const void* proj,
                       int32_t in_dtype, const void* conv_w, const void* dt_bias,

@@ -1543,6 +1543,21 @@ int kvc_state_ptrs(kvc_ctx* c, int32_t seq, int32_t ssm_layer, void** rec, void*
     return KVC_OK;
 }
 
+// Whether a launch takes the few-sequence matrix form.  Its three launches cost
+// more than one, and its state pass runs 64 workgroups per sequence, one per CU
+// at a time; the other kernels run 16 per sequence, token by token up to 12
+// tokens and in 6 us per 16-token block from 13.  us per layer, other kernel /
+// few-sequence form: 1 sequence, 8 tokens 15.8 / 17.5, 9 tokens 20.1 / 18.1,
+// 128 tokens 64.2 / 30.6, 500 tokens 206.6 / 58.0; 4 sequences, 9 tokens 20.9 /
+// 21.1, 12 tokens 24.6 / 21.6, 512 tokens 210 / 93; 5 sequences, 32 tokens
+// 29.5 / 30.0, 48 tokens 35.5 / 33.7; 7 sequences, 64 tokens 42.0 / 42.8, 96
+// tokens 54.8 / 53.2; 8 sequences, 512 tokens 210.5 / 206.9; 10 sequences 211.5
+// / 268.2.
+static bool deltanet_few(int32_t n_seqs, int32_t n_tok) {
+    if (n_seqs <= 4) return n_tok >= (n_seqs < 4 ? 9 : 10);
+    return n_seqs <= 7 && n_tok > kSsmChunk * (n_seqs - 3);
+}
+
 int kvc_deltanet_step(kvc_ctx* c, int32_t ssm_layer, const int32_t* seqs, int32_t n_seqs, int32_t n_tok,
                       const void* proj, int32_t in_dtype, const void* conv_w, const void* dt_bias, const void* a,
                       const void* norm_w, void* out, int32_t out_dtype, void* stream) {
@@ -1588,6 +1603,10 @@ int kvc_deltanet_step(kvc_ctx* c, int32_t ssm_layer, const int32_t* seqs, int32_
         d.n_tok = n_tok;
         d.ref_math = !(k.flags & KVC_FLAG_EXACT_MATH);
         for (int32_t j = 0; j < n; j++) d.slot[j] = seqs[i0 + j];
+        if (deltanet_few(n, n_tok)) {
+            d.ws = c->d_part;
+            d.seg_blocks = std::min((n_tok + kSsmChunk - 1) / kSsmChunk, kDnFewMax / (n * kSsmKHeads));
+        }
         int e = launch_deltanet(d, stream);
         if (e) return hip_err((hipError_t)e, "deltanet launch");
     }

@@ -184,8 +184,18 @@ struct DeltaNetArgs {
     int32_t n_tok;
     int32_t ref_math;       // 1: the reference's Schraudolph SiLU / sigmoid / softplus
     int32_t pad;
+    // few-sequence matrix form (ws not null): segments of seg_blocks 16-token
+    // blocks through the workspace, kDnFewBytes per (sequence, k-head, block)
+    void* ws;
+    int32_t seg_blocks;
+    int32_t seg_begin;      // set per segment by the launcher
+    int32_t seg_last;
+    int32_t pad2;
     int32_t slot[kMaxBatch];
 };
+constexpr int kSsmChunk = 16;       // tokens per block of the matrix forms
+constexpr int kDnFewBytes = 53248;
+constexpr int kDnFewMax = (int)(kPartBytes / kDnFewBytes);
 
 struct ZeroStateArgs {
     uint8_t* state;       // state pool base

@@ -2541,7 +2541,7 @@ void deltanet_kernel(DeltaNetArgs a) {
 // B fragment of a 4-token step j of the next product is then register j.
 // Tokens past the end of the last chunk enter as zero rows with beta = 0
 // and log decay 0, which leaves U, O and S unchanged.
-constexpr int kDnChunk = 16;
+constexpr int kDnChunk = kSsmChunk;
 // Calls of this many tokens or more run the matrix form (one partial block
 // below 16).  Measured at config e (64 sessions, interleaved): the blocked
 // kernel takes 84.0-85.4 / 89.9-90.2 us per layer at 12 / 13 tokens, the
@@ -3226,6 +3226,531 @@ void deltanet_mfma_kernel(DeltaNetArgs a) {
     conv_done();
 }
 
+// ---------------------------------------------------------------------------
+// Gated-DeltaNet in matrix form for calls of few sequences.  The persistent
+// kernel above runs one workgroup per (sequence, k-head): 16 for one sequence,
+// each of its 16-token blocks 6.1 us in series.  Of a block only the products
+// with the state depend on the block before, so three launches share the work:
+//   front  one workgroup per (k-head, block), all blocks at once: conv, gates,
+//          norms, T and M as above, then the state-free parts of the delta rule
+//          Uv = T diag(beta) V, Wk = T diag(beta e^g) K, into the workspace;
+//   state  one workgroup per (v-head, half of its 128 v-columns), block after
+//          block: U = Uv - Wk S^T, O = diag(e^g) Q S^T + M U,
+//          S^T <- e^{g_C} S^T + K^T diag(fc) U;
+//   norm   the gated RMSNorm of O, all blocks at once.
+// Rows of Wk are beta_t e^{g_t} k_t^T times a product of (I - beta k k^T), so
+// their entries stay below beta_t e^{g_t}: a power of two from that bound is
+// the row's scale for the two-part fp16 split (the other splits as above).
+// 500 tokens of one sequence: 206.6 -> 58.0 us per layer (front 15.4, state 35.9,
+// norm 6.8); the errors against a 64-bit result are no larger than the
+// persistent kernel's (fp32 outputs 2.5e-7 against 2.6e-7).
+//
+// Workspace of one (sequence, k-head, block), in 16-B pieces: Q's split
+// fragments and K^T's (kqf[1] and kt_pass's of the persistent kernel), then per
+// v-head Wk's split fragments, M as the A fragments of its four 4-token steps
+// [lane][step], the vectors [e^g, fc, 1 / Wk row scale][lane group][r] (token
+// 4 r + g) with e^{g_C}, and Uv [column tile][lane][r], replaced by O.
+constexpr int kDfQ = 0, kDfKt = 512, kDfHead = 1024;  // pieces
+constexpr int kDfWk = 0, kDfM = 512, kDfVec = 576, kDfUv = 640, kDfHeadSize = 1152;
+constexpr int kDfSize = kDfHead + 2 * kDfHeadSize;
+static_assert(kDfSize * 16 == kDnFewBytes, "workspace of one (sequence, k-head, block)");
+constexpr int kDfThreads = 512;
+
+// dn_split8 and dn_split4 (one scale) as one asm block, every dependent pair of
+// instructions at least two apart: a half-register write (mixlo / mixhi) costs
+// its consumer a wait state, and pair by pair the compiler puts an s_nop after
+// most of them.  Needs 12 more registers: the persistent kernel, at its limit,
+// spills and runs 268 us against 251 with it.
+__device__ __forceinline__ void dn_split8x(const float (&x)[8], float s, f16x8_t& h, f16x8_t& m) {
+    uint32_t h0, h1, h2, h3, m0, m1, m2, m3;
+    float r0, r1, r2, r3, r4, r5, r6, r7;
+    asm("v_fma_mixlo_f16 %0, %16, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %18, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %2, %20, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %3, %22, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %17, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %19, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %2, %21, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %3, %23, %24, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mix_f32 %8, %16, %24, -%0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %9, %17, %24, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %10, %18, %24, -%1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %11, %19, %24, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %12, %20, %24, -%2 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %13, %21, %24, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %14, %22, %24, -%3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %15, %23, %24, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_cvt_pkrtz_f16_f32 %4, %8, %9\n\t"
+        "v_cvt_pkrtz_f16_f32 %5, %10, %11\n\t"
+        "v_cvt_pkrtz_f16_f32 %6, %12, %13\n\t"
+        "v_cvt_pkrtz_f16_f32 %7, %14, %15"
+        : "=&v"(h0), "=&v"(h1), "=&v"(h2), "=&v"(h3), "=&v"(m0), "=&v"(m1), "=&v"(m2), "=&v"(m3), "=&v"(r0), "=&v"(r1),
+          "=&v"(r2), "=&v"(r3), "=&v"(r4), "=&v"(r5), "=&v"(r6), "=&v"(r7)
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(s));
+    h = __builtin_bit_cast(f16x8_t, u32x4{h0, h1, h2, h3});
+    m = __builtin_bit_cast(f16x8_t, u32x4{m0, m1, m2, m3});
+}
+__device__ __forceinline__ void dn_split4x(const float (&x)[4], float s, f16x4_t& h, f16x4_t& m) {
+    uint32_t h0, h1, m0, m1;
+    float r0, r1, r2, r3;
+    asm("v_fma_mixlo_f16 %0, %8, %12, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %10, %12, 0 op_sel_hi:[0,0,0]\n\t"
+        "s_nop 0\n\t"
+        "v_fma_mixhi_f16 %0, %9, %12, 0 op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %11, %12, 0 op_sel_hi:[0,0,0]\n\t"
+        "s_nop 0\n\t"
+        "v_fma_mix_f32 %4, %8, %12, -%0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %5, %9, %12, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %6, %10, %12, -%1 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mix_f32 %7, %11, %12, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_cvt_pkrtz_f16_f32 %2, %4, %5\n\t"
+        "v_cvt_pkrtz_f16_f32 %3, %6, %7"
+        : "=&v"(h0), "=&v"(h1), "=&v"(m0), "=&v"(m1), "=&v"(r0), "=&v"(r1), "=&v"(r2), "=&v"(r3)
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(s));
+    h = __builtin_bit_cast(f16x4_t, u32x2{h0, h1});
+    m = __builtin_bit_cast(f16x4_t, u32x2{m0, m1});
+}
+
+// A B^T of 16 rows of 128: a and b point at row c (the lane's), k = 32 g
+__device__ __forceinline__ f32x4 dn_gram(const float* a, const float* b) {
+    f32x4 a0 = {}, a1 = {};
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        const float4 x = *reinterpret_cast<const float4*>(a + 4 * m);
+        const float4 y = *reinterpret_cast<const float4*>(b + 4 * m);
+        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y.x, a0, 0, 0, 0);
+        a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y.y, a1, 0, 0, 0);
+        a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y.z, a0, 0, 0, 0);
+        a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y.w, a1, 0, 0, 0);
+    }
+    return a0 + a1;
+}
+
+template <bool BF16IN, bool REF>
+__global__ __launch_bounds__(kDfThreads) __attribute__((amdgpu_waves_per_eu(6, 8))) void deltanet_front_kernel(DeltaNetArgs a) {
+#pragma clang fp contract(off)
+    __shared__ float xs[kDnChunk][4 * 128 + 4];
+    __shared__ float lg[2][kDnChunk], gc[2][kDnChunk], bt[2][kDnChunk], be[2][kDnChunk];
+    __shared__ float lm[2][kDnChunk][kDnChunk];
+    __shared__ float sc[2][2][kDnChunk][kDnChunk];
+    const int item = blockIdx.x / a.seg_blocks;  // (sequence, k-head)
+    const int blk = blockIdx.x % a.seg_blocks + a.seg_begin;
+    const int seq = item / kSsmKHeads, kh = item % kSsmKHeads;
+    const int u = threadIdx.x, lane = u & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(u >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int tok0 = blk * kDnChunk, nb = min(kDnChunk, a.n_tok - tok0);
+    u32x4* ws = reinterpret_cast<u32x4*>(a.ws) + (size_t)blockIdx.x * kDfSize;
+    constexpr uint32_t kElt = BF16IN ? 2u : 4u;
+    const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(static_cast<const char*>(a.proj) + (size_t)seq * a.n_tok * kSsmProj * kElt), 0,
+        (int)((uint32_t)a.n_tok * (uint32_t)kSsmProj * kElt), 0x00020000);
+    auto row_off = [&](int tok) { return (uint32_t)max(min(tok, a.n_tok - 1), 0) * (uint32_t)kSsmProj * kElt; };
+    constexpr uint32_t kAlpha = kSsmC + kSsmVHeads * kSsmDv, kBeta = kAlpha + kSsmVHeads;
+
+    // conv + SiLU of channel u; the window before the block is the call's
+    // earlier rows, or the conv state at its start
+    {
+        const int ch = dn_channel(u, kh);
+        uint32_t xin[kDnChunk], xw[3];
+#pragma unroll
+        for (int i = 0; i < kDnChunk; i++) xin[i] = load_raw_buf<BF16IN>(prs, (uint32_t)ch * kElt, row_off(tok0 + i));
+#pragma unroll
+        for (int i = 0; i < 3; i++) xw[i] = load_raw_buf<BF16IN>(prs, (uint32_t)ch * kElt, row_off(tok0 - 3 + i));
+        const float4 cw = make_float4(a.conv_w[ch], a.conv_w[kSsmC + ch], a.conv_w[2 * kSsmC + ch], a.conv_w[3 * kSsmC + ch]);
+        const float* conv = reinterpret_cast<const float*>(a.state + (size_t)a.slot[seq] * a.state_bytes + a.layer_off +
+                                                           a.rec_bytes);
+        float w0 = conv[ch], w1 = conv[kSsmC + ch], w2 = conv[2 * kSsmC + ch];
+        if (blk > 0) {
+            w0 = raw_f<BF16IN>(xw[0]);
+            w1 = raw_f<BF16IN>(xw[1]);
+            w2 = raw_f<BF16IN>(xw[2]);
+        }
+        // gate pair of wave 7: token ab_t, v-head kh + 16 ab_h
+        const int ab_t = (lane >> 1) & (kDnChunk - 1), ab_h = lane & 1, vh = kh + kSsmKHeads * ab_h;
+        float alpha = 0.f, braw = 0.f, dtb = 0.f, av = 0.f;
+        if (wave == 7) {
+            const uint32_t ro = (uint32_t)min(ab_t, nb - 1) * (uint32_t)kSsmProj * kElt;
+            alpha = raw_f<BF16IN>(load_raw_buf<BF16IN>(prs, ro + (kAlpha + (uint32_t)vh) * kElt, row_off(tok0)));
+            braw = raw_f<BF16IN>(load_raw_buf<BF16IN>(prs, ro + (kBeta + (uint32_t)vh) * kElt, row_off(tok0)));
+            dtb = a.dt_bias[vh];
+            av = a.a[vh];
+        }
+#pragma unroll
+        for (int i = 0; i < kDnChunk; i++) {
+            const float xv = raw_f<BF16IN>(xin[i]);
+            float sum = w0 * cw.x;
+            sum = fmaf(w1, cw.y, sum);
+            sum = fmaf(w2, cw.z, sum);
+            sum = fmaf(xv, cw.w, sum);
+            xs[i][u] = i < nb ? dn_silu<REF>(sum) : 0.f;
+            w0 = w1;
+            w1 = w2;
+            w2 = xv;
+        }
+        if (wave == 7 && lane < 2 * kDnChunk) {
+            const float biased = alpha + dtb;
+            const float ex = REF ? schraudolph_exp(biased) : dn_exp(biased);
+            const float sp = biased > 20.0f ? biased : dn_log(1.0f + ex);
+            lg[ab_h][ab_t] = ab_t < nb ? sp * av : 0.f;
+            bt[ab_h][ab_t] = ab_t < nb ? dn_beta<REF>(braw) : 0.f;
+        }
+    }
+    lds_barrier();
+    if (wave < 4) {  // q / k norms of token 4 wave + g, in place
+        const int tk = 4 * wave + g, col0 = c * 4;
+        float qv[kDnCols], kv[kDnCols];
+        dn_qk(xs[tk], col0, a.eps, qv, kv);
+        if (tk < nb) {
+#pragma unroll
+            for (int j = 0; j < kDnCols; j += 4) {
+                const int cc = col0 + (j ? kSsmDk / 2 : 0);
+                *reinterpret_cast<float4*>(&xs[tk][cc]) = make_float4(qv[j], qv[j + 1], qv[j + 2], qv[j + 3]);
+                *reinterpret_cast<float4*>(&xs[tk][128 + cc]) = make_float4(kv[j], kv[j + 1], kv[j + 2], kv[j + 3]);
+            }
+        }
+    } else if (wave == 4 && lane < 2 * kDnChunk) {  // prefix sums of token tk, v-head h
+        const int h = lane >> 4, tk = lane & 15;
+        float run = 0.f, all = 0.f;
+#pragma unroll
+        for (int i = 0; i < kDnChunk; i++) {
+            const float v = lg[h][i];
+            all += v;
+            run = i <= tk ? all : run;
+        }
+        const float e = dn_exp(run), b = bt[h][tk] * e;
+        const int eb = min(max((int)(__float_as_uint(b) >> 23), 29), 254);
+        gc[h][tk] = run;
+        be[h][tk] = b;
+        float* vec = reinterpret_cast<float*>(ws + kDfHead + h * kDfHeadSize + kDfVec);
+        const int at = (tk & 3) * 4 + (tk >> 2);
+        vec[at] = e;
+        vec[16 + at] = dn_exp(all - run);
+        vec[32 + at] = __uint_as_float((uint32_t)(eb - 13) << 23);  // 1 / the row's scale 2^(140 - eb)
+        if (tk == kDnChunk - 1) vec[48] = e;
+    }
+    lds_barrier();
+    if (wave < 2) {
+        // T of v-head `wave` (as the persistent kernel, N formed from the
+        // wave's own K K^T: lane (g, c) holds rows 4 g + r of column c)
+        float(*n1)[kDnChunk] = lm[wave];
+        float(*n2)[kDnChunk] = sc[wave][0];
+        float(*n4)[kDnChunk] = sc[wave][1];
+        float(*xm)[kDnChunk] = sc[wave][0];  // N^2 is dead once X is formed
+        f32x4 pr = dn_gram(&xs[c][128 + 32 * g], &xs[c][128 + 32 * g]);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int ti = 4 * g + r;
+            const float dg = dn_exp(gc[wave][ti] - gc[wave][c]);
+            n1[ti][c] = c < ti ? bt[wave][ti] * (dg * pr[r]) : 0.f;
+        }
+        pr = dn_m16(n1, n1, g, c);
+#pragma unroll
+        for (int r = 0; r < 4; r++) n2[4 * g + r][c] = pr[r];
+        pr = dn_m16(n2, n2, g, c);
+#pragma unroll
+        for (int r = 0; r < 4; r++) n4[4 * g + r][c] = pr[r];
+        pr = dn_m16(n1, n2, g, c);  // X = I - N + N^2 - N N^2
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            xm[4 * g + r][c] = ((4 * g + r == c) ? 1.f : 0.f) - n1[4 * g + r][c] + n2[4 * g + r][c] - pr[r];
+        pr = dn_m16(n4, n4, g, c);
+#pragma unroll
+        for (int r = 0; r < 4; r++) n1[4 * g + r][c] = pr[r];  // N^8
+        pr = dn_m16(xm, n4, g, c);  // X <- X + X N^4
+#pragma unroll
+        for (int r = 0; r < 4; r++) xm[4 * g + r][c] += pr[r];
+        pr = dn_m16(xm, n1, g, c);  // T = X + X N^8
+#pragma unroll
+        for (int r = 0; r < 4; r++) n1[4 * g + r][c] = xm[4 * g + r][c] + pr[r];
+    } else if (wave < 4) {
+        // M of v-head wave - 2 from K Q^T with both operands' rows in sigma
+        // order: lane (g, c), register j holds Q.K of token sigma(c) with 4 j + g
+        const int h = wave - 2, ti = dn_sigma(c);
+        f32x4 m = dn_gram(&xs[ti][128 + 32 * g], &xs[ti][32 * g]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int si = 4 * j + g;
+            const float dg = dn_exp(gc[h][ti] - gc[h][si]);
+            m[j] = si <= ti ? dg * m[j] : 0.f;
+        }
+        ws[kDfHead + h * kDfHeadSize + kDfM + lane] = __builtin_bit_cast(u32x4, m);
+    } else {
+        // Q's split fragments of 32-k step ks, K^T's of 16-row fragments 2 ks, 2 ks + 1
+        const int ks = wave - 4;
+        const float* row = &xs[dn_sigma(c)][32 * ks + 4 * g];
+        const float4 x0 = *reinterpret_cast<const float4*>(row);
+        const float4 x1 = *reinterpret_cast<const float4*>(row + 16);
+        const float v8[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        f16x8_t h, m;
+        dn_split8x(v8, 16384.f, h, m);
+        ws[kDfQ + ((ks * 4 + g) * 2) * 16 + c] = __builtin_bit_cast(u32x4, h);
+        ws[kDfQ + ((ks * 4 + g) * 2 + 1) * 16 + c] = __builtin_bit_cast(u32x4, m);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int f = 2 * ks + i;
+            const float kv[4] = {xs[g][128 + 16 * f + c], xs[4 + g][128 + 16 * f + c], xs[8 + g][128 + 16 * f + c],
+                                 xs[12 + g][128 + 16 * f + c]};
+            f16x4_t kh4, km4;
+            dn_split4x(kv, 16384.f, kh4, km4);
+            const u32x2 hw = __builtin_bit_cast(u32x2, kh4), mw = __builtin_bit_cast(u32x2, km4);
+            ws[kDfKt + f * 64 + lane] = u32x4{hw[0], hw[1], mw[0], mw[1]};
+        }
+    }
+    lds_barrier();
+    // v-head h: Uv's column tiles 2 ks and 2 ks + 1, and the same k rows of
+    // Wk^T = K^T (T diag(beta e^g))^T, whose result registers are Wk's fragment
+    // of 32-k step ks as they stand (lane (g, c): token sigma(c), k = 16 vt +
+    // 4 g + e)
+    const int h = wave >> 2, ks = wave & 3, tk = dn_sigma(c);
+    float tr[4], bk[4], bv[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        tr[j] = lm[h][tk][4 * j + g];
+        bk[j] = tr[j] * be[h][4 * j + g];
+        bv[j] = bt[h][4 * j + g];
+    }
+    float v8[8];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int vt = 2 * ks + i, col = 16 * vt + c;
+        f32x4 w = {}, v = {};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            w = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[4 * j + g][128 + col], bk[j], w, 0, 0, 0);
+            v = __builtin_amdgcn_mfma_f32_16x16x4f32(tr[j], bv[j] * xs[4 * j + g][256 + 128 * h + col], v, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) v8[4 * i + e] = w[e];
+        ws[kDfHead + h * kDfHeadSize + kDfUv + vt * 64 + lane] = __builtin_bit_cast(u32x4, v);
+    }
+    const int eb = min(max((int)(__float_as_uint(be[h][tk]) >> 23), 29), 254);
+    f16x8_t hh, hm;
+    dn_split8x(v8, __uint_as_float((uint32_t)(267 - eb) << 23), hh, hm);
+    u32x4* dst = ws + kDfHead + h * kDfHeadSize + kDfWk + ((ks * 4 + g) * 2) * 16 + c;
+    dst[0] = __builtin_bit_cast(u32x4, hh);
+    dst[16] = __builtin_bit_cast(u32x4, hm);
+}
+
+// State pass: wave w < 4 of (sequence, v-head, half) holds v-columns
+// 64 half + 16 w .. +15 as the persistent kernel's state fragments
+// (st[m] = S^T[16 m + 4 g .. +3][column c]).  Waves 4 and 5 copy the blocks'
+// operands into kDfBufs LDS buffers, kDfBufs - 1 blocks ahead (LDS DMA,
+// kDfCopies per wave and block, always issued: past the end the last block
+// again); they wait for copies by count, and one barrier per block both
+// publishes the next block's buffer and frees the one before.
+// What bounds it: the block chain of a wave alone on its SIMD, which issues an
+// instruction per 5 cycles and an MFMA per 16 (state splits 80 instructions, 40
+// MFMAs, 32 multiply-adds of the update): 0.96 us per block, 1.45 with the
+// copies in these waves and every fragment read where it is used (leaving the
+// copies out altogether changes nothing).  So fragments are read from LDS during the block
+// before, part products have accumulators of their own, and both cross terms
+// of the update share an MFMA.  Two waves per tile, 64 k rows each, exchanging
+// their parts of Wk S^T through LDS, were no faster (1.18 us per block: the
+// second barrier and the work on U done twice).
+constexpr int kDfBufs = 5, kDfCopyWaves = 2, kDfCopies = 30 / kDfCopyWaves;
+constexpr int kDfStateThreads = 64 * (4 + kDfCopyWaves);
+constexpr int kDfBufQ = 0, kDfBufKt = 512, kDfBufWk = 1024, kDfBufMv = 1536, kDfBufUv = 1664, kDfBufSize = 1920;
+template <bool BF16IN>
+__global__ __launch_bounds__(kDfStateThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void deltanet_state_kernel(DeltaNetArgs a) {
+#pragma clang fp contract(off)
+    __shared__ u32x4 buf[kDfBufs][kDfBufSize];
+    const int half = blockIdx.x & 1, vh = (blockIdx.x >> 1) % kSsmVHeads, seq = (blockIdx.x >> 1) / kSsmVHeads;
+    const int kh = vh % kSsmKHeads, h = vh / kSsmKHeads;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, c = lane & 15;
+    const int nblk = a.seg_blocks;
+    char* ws = reinterpret_cast<char*>(a.ws) + (size_t)(seq * kSsmKHeads + kh) * nblk * kDnFewBytes;
+    if (wave >= 4) {
+        const uint32_t lds0 = lds_addr(&buf[0][0]), lo = (uint32_t)lane * 16;
+        auto issue = [&](int b) {
+            const char* src = ws + (size_t)min(b, nblk - 1) * kDnFewBytes;
+            const uint32_t dst = lds0 + (uint32_t)(b % kDfBufs) * (kDfBufSize * 16);
+#pragma unroll
+            for (int j = 0; j < kDfCopies; j++) {
+                // 1 KiB per copy: Q, K^T (16), Wk, M, vectors (10), this half's Uv (4)
+                const int i = wave - 4 + kDfCopyWaves * j;
+                const int at = i + (i < 16 ? 0 : h * (kDfHeadSize / 64)) + (i < 26 ? 0 : 4 * half);
+                lds_dma16s(src + at * 1024, lo, dst + i * 1024);
+            }
+        };
+        for (int b = 0; b < kDfBufs - 1; b++) issue(b);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kDfBufs - 2) * kDfCopies) : "memory");  // block 0 is in
+        for (int b = 0; b < nblk; b++) {
+            // blocks b and b + 1 are in
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((kDfBufs - 3) * kDfCopies) : "memory");
+            issue(b + kDfBufs - 1);
+        }
+        __builtin_amdgcn_s_waitcnt(0);  // no copy may still write LDS when the wave ends
+        return;
+    }
+    float* S = reinterpret_cast<float*>(a.state + (size_t)a.slot[seq] * a.state_bytes + a.layer_off) +
+               ((size_t)vh * kSsmDv + 64 * half + 16 * wave + c) * kSsmDk + 4 * g;
+    f32x4 st[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) st[m] = *reinterpret_cast<const f32x4*>(S + 16 * m);
+    float smax = 0.f;
+#pragma unroll
+    for (int m = 0; m < 8; m++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) smax = fmaxf(smax, fabsf(st[m][e]));
+    smax = max_xor32(max_xor16(smax));
+    float dk = 1.f;  // the registers hold S^T / dk (as in the persistent kernel)
+    char* wso = ws + (kDfHead + h * kDfHeadSize + kDfUv) * 16 + ((4 * half + wave) * 64 + lane) * 16;
+    // a block's operands
+    u32x4 fw[4][2], fq[4][2], fk[8];
+    f32x4 uv0, wsc, fc, eg, mf;
+    float egc;
+    auto read_a = [&](const u32x4* B) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                fw[ks][q] = B[kDfBufWk + (ks * 4 + g) * 32 + 16 * q + c];
+                fq[ks][q] = B[kDfBufQ + (ks * 4 + g) * 32 + 16 * q + c];
+            }
+    };
+    auto read_b = [&](const u32x4* B) {
+        const float* vec = reinterpret_cast<const float*>(B + kDfBufMv + 64);
+        egc = vec[48];
+        uv0 = __builtin_bit_cast(f32x4, B[kDfBufUv + wave * 64 + lane]);
+        wsc = *reinterpret_cast<const f32x4*>(vec + 32 + 4 * g);
+        fc = *reinterpret_cast<const f32x4*>(vec + 16 + 4 * g);
+#pragma unroll
+        for (int m = 0; m < 8; m++) fk[m] = B[kDfBufKt + m * 64 + lane];
+        eg = *reinterpret_cast<const f32x4*>(vec + 4 * g);
+        mf = __builtin_bit_cast(f32x4, B[kDfBufMv + lane]);
+    };
+    lds_barrier();
+    read_a(buf[0]);
+    read_b(buf[0]);
+    for (int b = 0; b < nblk; b++) {
+        lds_barrier();
+        const u32x4* Bn = buf[(b + 1) % kDfBufs];
+        const int ex = min(max((int)(__float_as_uint(smax) >> 23), 29), 254);
+        const float ssc = __uint_as_float((uint32_t)(268 - ex) << 23);       // 2^(141 - ex)
+        const float sinv = __uint_as_float((uint32_t)(ex - 14) << 23) * dk;  // dk / ssc
+        // W1 = Wk S^T and W2 = Q S^T
+        f32x4 w1[3] = {}, w2[3] = {};
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            const float sv[8] = {st[2 * ks][0],     st[2 * ks][1],     st[2 * ks][2],     st[2 * ks][3],
+                                 st[2 * ks + 1][0], st[2 * ks + 1][1], st[2 * ks + 1][2], st[2 * ks + 1][3]};
+            f16x8_t sh, sm;
+            dn_split8x(sv, ssc, sh, sm);
+            const f16x8_t wh = __builtin_bit_cast(f16x8_t, fw[ks][0]), wm = __builtin_bit_cast(f16x8_t, fw[ks][1]);
+            const f16x8_t qh = __builtin_bit_cast(f16x8_t, fq[ks][0]), qm = __builtin_bit_cast(f16x8_t, fq[ks][1]);
+            w1[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wm, sh, w1[0], 0, 0, 0);
+            w1[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh, sm, w1[1], 0, 0, 0);
+            w1[2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh, sh, w1[2], 0, 0, 0);
+            w2[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qm, sh, w2[0], 0, 0, 0);
+            w2[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh, sm, w2[1], 0, 0, 0);
+            w2[2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh, sh, w2[2], 0, 0, 0);
+        }
+        const float dkn = dk * egc;
+        const bool fold = !(dkn >= 0x1p-80f);  // uniform
+        const float rdk = fold ? 1.f : 1.f / dkn;
+        read_a(Bn);
+        const f32x4 us4 = wsc * sinv;
+        f32x4 uu;
+#pragma unroll
+        for (int r = 0; r < 4; r++) uu[r] = uv0[r] - ((w1[0][r] + w1[1][r]) + w1[2][r]) * us4[r];
+        const float uv[4] = {uu[0] * fc[0], uu[1] * fc[1], uu[2] * fc[2], uu[3] * fc[3]};
+        float mu = fmaxf(fmaxf(fabsf(uv[0]), fabsf(uv[1])), fmaxf(fabsf(uv[2]), fabsf(uv[3])));
+        mu = max_xor32(max_xor16(mu));
+        const int eu = min(max((int)(__float_as_uint(mu) >> 23), 29), 254);
+        f16x4_t uh, um;
+        dn_split4x(uv, __uint_as_float((uint32_t)(268 - eu) << 23), uh, um);
+        const float uinv = __uint_as_float((uint32_t)(eu - 28) << 23) * rdk;
+        if (__builtin_amdgcn_ballot_w64(fold) != 0) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) st[m] *= dkn;
+        }
+        // K^T (diag(fc) U): both cross terms kh um + km uh in one 32-deep MFMA,
+        // [kh km] against [um uh], then kh uh
+        const u32x2 uhw = __builtin_bit_cast(u32x2, uh), umw = __builtin_bit_cast(u32x2, um);
+        const f16x8_t ux = __builtin_bit_cast(f16x8_t, u32x4{umw[0], umw[1], uhw[0], uhw[1]});
+        f32x4 t[8], o;
+#pragma unroll
+        for (int m = 0; m < 8; m++)
+            t[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, fk[m]), ux, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < 8; m++)
+            t[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4_t, u32x2{fk[m][0], fk[m][1]}), uh, t[m], 0, 0, 0);
+        smax = fold ? fmaf(16.f, mu, dkn * smax) : fmaf(16.f * mu, rdk, smax);
+        dk = fold ? 1.f : dkn;
+#pragma unroll
+        for (int r = 0; r < 4; r++) o[r] = eg[r] * (((w2[0][r] + w2[1][r]) + w2[2][r]) * (sinv * 0x1p-14f));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            o = __builtin_amdgcn_mfma_f32_16x16x4f32(mf[j], uu[j], o, 0, 0, 0);
+#pragma unroll
+            for (int m = 2 * j; m < 2 * j + 2; m++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) st[m][e] = fmaf(t[m][e], uinv, st[m][e]);
+        }
+        read_b(Bn);
+        *reinterpret_cast<f32x4*>(wso) = o * a.out_scale;
+        wso += kDnFewBytes;
+    }
+#pragma unroll
+    for (int m = 0; m < 8; m++) *reinterpret_cast<f32x4*>(S + 16 * m) = st[m] * dk;
+    if (a.seg_last && h == 0) {  // the conv window of the k-head's channels: the call's last three rows
+        float* conv = reinterpret_cast<float*>(a.state + (size_t)a.slot[seq] * a.state_bytes + a.layer_off + a.rec_bytes);
+        const int ch = dn_channel(256 * half + threadIdx.x, kh);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            conv[(size_t)i * kSsmC + ch] = load_f<BF16IN>(a.proj, ((size_t)seq * a.n_tok + a.n_tok - 3 + i) * kSsmProj + ch);
+    }
+}
+
+// Gated RMSNorm of O: one wave per (sequence, k-head, block, v-head); lane
+// (g, c) holds tokens 4 r + g of columns 16 vt + c.
+template <bool BF16IN, bool REF>
+__global__ __launch_bounds__(256) void deltanet_norm_kernel(DeltaNetArgs a) {
+#pragma clang fp contract(off)
+    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int h = w & 1, ib = w >> 1;
+    const int item = ib / a.seg_blocks, blk = ib % a.seg_blocks + a.seg_begin;
+    const int seq = item / kSsmKHeads, vh = item % kSsmKHeads + kSsmKHeads * h;
+    const f32x4* src = reinterpret_cast<const f32x4*>(a.ws) + (size_t)ib * kDfSize + kDfHead + h * kDfHeadSize + kDfUv + lane;
+    const int tok0 = blk * kDnChunk + g;
+    size_t zrow[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        zrow[r] = ((size_t)seq * a.n_tok + min(tok0 + 4 * r, a.n_tok - 1)) * kSsmProj + kSsmC + (size_t)vh * kSsmDv + c;
+    f32x4 o[8];
+    uint32_t z[8][4];
+    float nw[8];
+#pragma unroll
+    for (int vt = 0; vt < 8; vt++) {
+        o[vt] = src[vt * 64];
+        nw[vt] = a.norm_w[16 * vt + c];
+#pragma unroll
+        for (int r = 0; r < 4; r++) z[vt][r] = load_raw<BF16IN>(a.proj, zrow[r] + 16 * vt);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float ss = 0.f;
+#pragma unroll
+        for (int vt = 0; vt < 8; vt++) ss = fmaf(o[vt][r], o[vt][r], ss);
+        const float rms = dn_rsqrt(sum16(ss) / kSsmDv + a.eps);
+        const int tok = tok0 + 4 * r;
+        if (tok >= a.n_tok) continue;
+        const size_t oi = ((size_t)seq * a.n_tok + tok) * (kSsmVHeads * kSsmDv) + (size_t)vh * kSsmDv + c;
+#pragma unroll
+        for (int vt = 0; vt < 8; vt++) {
+            const float y = o[vt][r] * rms * nw[vt] * dn_silu<REF>(raw_f<BF16IN>(z[vt][r]));
+            if (a.out_bf16)
+                static_cast<uint16_t*>(a.out)[oi + 16 * vt] = (uint16_t)f32_to_bf16_rne(y);
+            else
+                static_cast<float*>(a.out)[oi + 16 * vt] = y;
+        }
+    }
+}
+
 constexpr int kDnPf = 4;  // rows loaded ahead in the streaming kernel (2, 6 and 8 measured slower)
 
 template <bool BF16IN, bool REF>
@@ -3650,6 +4175,24 @@ static void launch_deltanet_t(const DeltaNetArgs& a, hipStream_t stream) {
             hipLaunchKernelGGL((deltanet_decode_kernel<true, REF>), grid, block, 0, stream, a);
         else
             hipLaunchKernelGGL((deltanet_decode_kernel<false, REF>), grid, block, 0, stream, a);
+    } else if (a.ws) {  // few sequences: front, state and norm passes per segment of blocks
+        DeltaNetArgs d = a;
+        const int nblk = (a.n_tok + kDnChunk - 1) / kDnChunk, items = a.n_seqs * kSsmKHeads;
+        for (int b = 0; b < nblk; b += a.seg_blocks) {
+            d.seg_begin = b;
+            d.seg_blocks = std::min(a.seg_blocks, nblk - b);
+            d.seg_last = b + d.seg_blocks == nblk;
+            const dim3 fgrid(items * d.seg_blocks), sgrid(a.n_seqs * kSsmVHeads * 2), ngrid(items * d.seg_blocks / 2);
+            if (a.in_bf16) {
+                hipLaunchKernelGGL((deltanet_front_kernel<true, REF>), fgrid, dim3(kDfThreads), 0, stream, d);
+                hipLaunchKernelGGL((deltanet_state_kernel<true>), sgrid, dim3(kDfStateThreads), 0, stream, d);
+                hipLaunchKernelGGL((deltanet_norm_kernel<true, REF>), ngrid, dim3(256), 0, stream, d);
+            } else {
+                hipLaunchKernelGGL((deltanet_front_kernel<false, REF>), fgrid, dim3(kDfThreads), 0, stream, d);
+                hipLaunchKernelGGL((deltanet_state_kernel<false>), sgrid, dim3(kDfStateThreads), 0, stream, d);
+                hipLaunchKernelGGL((deltanet_norm_kernel<false, REF>), ngrid, dim3(256), 0, stream, d);
+            }
+        }
     } else if (a.n_tok >= kDnMatrixMin) {
         // persistent: at most one workgroup per CU (its LDS needs a CU); the
         // CU count of the current device is looked up once per process
