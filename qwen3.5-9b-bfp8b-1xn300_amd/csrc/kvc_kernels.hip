@@ -3753,9 +3753,18 @@ __global__ __launch_bounds__(256) void deltanet_norm_kernel(DeltaNetArgs a) {
 
 constexpr int kDnPf = 4;  // rows loaded ahead in the streaming kernel (2, 6 and 8 measured slower)
 
-template <bool BF16IN, bool REF>
-__global__ __launch_bounds__(kDnThreads) void deltanet_decode_kernel(DeltaNetArgs a) {
+// THREADS = 512, a lane holding 8 state rows, 4 of them ahead; or 1024 for
+// launches that leave CUs idle anyway, a lane holding 4 rows, all requested at
+// entry: the rows' chain is half as long and no load waits for another (the
+// arithmetic and its order are the same).  One sequence 7.06 -> 6.37 us per
+// layer, four 8.55 -> 6.91.
+template <bool BF16IN, bool REF, int THREADS>
+__global__ __launch_bounds__(THREADS) void deltanet_decode_kernel(DeltaNetArgs a) {
 #pragma clang fp contract(off)
+    constexpr int kHeadWaves = THREADS / 128;          // waves per v-head
+    constexpr int kWaveRows = kSsmDv / kHeadWaves;     // state rows per wave
+    constexpr int kRows = kWaveRows / 4;               // per lane
+    static_assert(kRows >= kDnPf, "the rows requested at entry");
     __shared__ float conv_lds[4 * 128];
     __shared__ float o_lds[2][kSsmDv];
     const int b = blockIdx.x;
@@ -3763,10 +3772,10 @@ __global__ __launch_bounds__(kDnThreads) void deltanet_decode_kernel(DeltaNetArg
     const int kh = b - s * kSsmKHeads;
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
-    const int vl = wave >> 2, wi = wave & 3;
+    const int vl = wave / kHeadWaves, wi = wave % kHeadWaves;
     const int vh = kh + kSsmKHeads * vl;
     const int rg = lane >> 4, col0 = (lane & 15) * 4;
-    const int rbase = wi * 32 + rg;
+    const int rbase = wi * kWaveRows + rg;
 
     uint8_t* slot = a.state + (size_t)a.slot[s] * a.state_bytes + a.layer_off;
     float* S = reinterpret_cast<float*>(slot) + (size_t)vh * kSsmDv * kSsmDk + col0;
@@ -3779,33 +3788,40 @@ __global__ __launch_bounds__(kDnThreads) void deltanet_decode_kernel(DeltaNetArg
         buf[p][0] = nt_ld4(src);
         buf[p][1] = nt_ld4(src + kSsmDk / 2);
     }
-    const int ch = dn_channel(t, kh);
     const size_t prow = (size_t)s * kSsmProj;
     constexpr size_t kZ = kSsmC, kAlpha = kSsmC + kSsmVHeads * kSsmDv, kBeta = kAlpha + kSsmVHeads;
-    const int zd = wi * 32 + (lane & 31);
+    const bool owns = THREADS == 512 || t < 512;       // thread t < 512 owns conv channel t
+    const bool writes = THREADS == 512 || wi < 4;      // waves that write 32 output dims of the v-head
+    const int ch = dn_channel(t & 511, kh);
+    const int zd = (wi & 3) * 32 + (lane & 31);
     const float x = load_f<BF16IN>(a.proj, prow + ch);
     const float z = load_f<BF16IN>(a.proj, prow + kZ + (size_t)vh * kSsmDv + zd);
     const float alpha = load_f<BF16IN>(a.proj, prow + kAlpha + vh);
     const float braw = load_f<BF16IN>(a.proj, prow + kBeta + vh);
-    const float c0 = conv[ch], c1 = conv[kSsmC + ch], c2 = conv[2 * kSsmC + ch];
-    float sum = c0 * a.conv_w[ch];
-    sum = fmaf(c1, a.conv_w[kSsmC + ch], sum);
-    sum = fmaf(c2, a.conv_w[2 * kSsmC + ch], sum);
-    sum = fmaf(x, a.conv_w[3 * kSsmC + ch], sum);
-    conv_lds[t] = dn_silu<REF>(sum);
-    conv[ch] = c1;
-    conv[kSsmC + ch] = c2;
-    conv[2 * kSsmC + ch] = x;
-    __syncthreads();
+    if (owns) {
+        const float c0 = conv[ch], c1 = conv[kSsmC + ch], c2 = conv[2 * kSsmC + ch];
+        float sum = c0 * a.conv_w[ch];
+        sum = fmaf(c1, a.conv_w[kSsmC + ch], sum);
+        sum = fmaf(c2, a.conv_w[2 * kSsmC + ch], sum);
+        sum = fmaf(x, a.conv_w[3 * kSsmC + ch], sum);
+        conv_lds[t] = dn_silu<REF>(sum);
+        conv[ch] = c1;
+        conv[kSsmC + ch] = c2;
+        conv[2 * kSsmC + ch] = x;
+    }
+    if constexpr (THREADS == 512)
+        __syncthreads();
+    else
+        lds_barrier();  // without a wait for the conv stores
 
     float q[kDnCols], k[kDnCols], decay, beta;
     dn_qk(conv_lds, col0, a.eps, q, k);
     dn_gates<REF>(alpha, braw, a.dt_bias[vh], a.a[vh], decay, beta);
 #pragma unroll
-    for (int r = 0; r < kDnRows; r++) {
+    for (int r = 0; r < kRows; r++) {
         float st[kDnCols] = {buf[r % kDnPf][0].x, buf[r % kDnPf][0].y, buf[r % kDnPf][0].z, buf[r % kDnPf][0].w,
                              buf[r % kDnPf][1].x, buf[r % kDnPf][1].y, buf[r % kDnPf][1].z, buf[r % kDnPf][1].w};
-        if (r + kDnPf < kDnRows) {
+        if (r + kDnPf < kRows) {
             const float* src = S + (size_t)(rbase + 4 * (r + kDnPf)) * kSsmDk;
             buf[r % kDnPf][0] = nt_ld4(src);
             buf[r % kDnPf][1] = nt_ld4(src + kSsmDk / 2);
@@ -3815,8 +3831,11 @@ __global__ __launch_bounds__(kDnThreads) void deltanet_decode_kernel(DeltaNetArg
         nt_st4(dst, st[0], st[1], st[2], st[3]);
         nt_st4(dst + kSsmDk / 2, st[4], st[5], st[6], st[7]);
     }
-    __syncthreads();
-    dn_norm_out<REF>(a, o_lds[vl], lane, wi, vh, (size_t)s * (kSsmVHeads * kSsmDv), z);
+    if constexpr (THREADS == 512)
+        __syncthreads();
+    else
+        lds_barrier();
+    if (writes) dn_norm_out<REF>(a, o_lds[vl], lane, wi, vh, (size_t)s * (kSsmVHeads * kSsmDv), z);
 }
 
 // ---------------------------------------------------------------------------
@@ -4171,10 +4190,17 @@ template <bool REF>
 static void launch_deltanet_t(const DeltaNetArgs& a, hipStream_t stream) {
     const dim3 grid(a.n_seqs * kSsmKHeads), block(kDnThreads);
     if (a.n_tok == 1) {
-        if (a.in_bf16)
-            hipLaunchKernelGGL((deltanet_decode_kernel<true, REF>), grid, block, 0, stream, a);
+        // up to one 1024-thread workgroup per CU: 16 sequences 14.9 -> 13.2 us,
+        // 24 the same, 32 26.4 -> 28.2
+        const bool wide = a.n_seqs * kSsmKHeads <= 256;
+        if (wide && a.in_bf16)
+            hipLaunchKernelGGL((deltanet_decode_kernel<true, REF, 1024>), grid, dim3(1024), 0, stream, a);
+        else if (wide)
+            hipLaunchKernelGGL((deltanet_decode_kernel<false, REF, 1024>), grid, dim3(1024), 0, stream, a);
+        else if (a.in_bf16)
+            hipLaunchKernelGGL((deltanet_decode_kernel<true, REF, 512>), grid, block, 0, stream, a);
         else
-            hipLaunchKernelGGL((deltanet_decode_kernel<false, REF>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((deltanet_decode_kernel<false, REF, 512>), grid, block, 0, stream, a);
     } else if (a.ws) {  // few sequences: front, state and norm passes per segment of blocks
         DeltaNetArgs d = a;
         const int nblk = (a.n_tok + kDnChunk - 1) / kDnChunk, items = a.n_seqs * kSsmKHeads;
