@@ -1087,19 +1087,50 @@ int kvc_qkv_append(kvc_ctx* c, int32_t layer, const int32_t* seqs, int32_t n_seq
     return KVC_OK;
 }
 
-// Decode launches with fewer work items than this split each chunk's output
-// dims over 2 workgroups (one per CU of the 256 is the aim).
-constexpr int64_t kDsplitBelowItems = 256;
-
-static int32_t auto_chunk_blocks(kvc_ctx* c, int64_t total_blocks) {
-    if (c->cfg.decode_chunk_blocks > 0) return c->cfg.decode_chunk_blocks;
-    // About 16 items per CU on 256 CUs (kAutoItems): three decode workgroups
-    // are resident per CU, and many short items balance the ragged sequences'
-    // chunks better than a few long ones (config d: 598-602 us per layer at
-    // 3072-6144 items against 627 at 1024).  Chunks of at least 4 blocks keep
-    // the split-K partial traffic and the final combine small.
-    int64_t cb = (total_blocks * kKvHeads + kAutoItems - 1) / kAutoItems;
-    return (int32_t)std::max<int64_t>(4, cb);
+// Blocks per split-K chunk when the caller leaves it open, from the sequences'
+// block counts nb[n].  Two ways to cut a launch:
+//  - one workgroup per CU (at most 64 chunks x 4 heads, 32 chunks per
+//    sequence for a short combine): the CUs share HBM, so it takes the time of
+//    its bytes plus what the longest chunk has over the mean, at 0.45 us per
+//    block of a workgroup alone;
+//  - short chunks in many rounds, which balance ragged sequences: an item costs
+//    7 ns of the launch's time, the last one of a CU 0.45 us per block, least
+//    at 0.25 sqrt(total blocks) per chunk.
+// The cheaper by that estimate is taken.  us per layer of kvc_decode_step, the
+// former rule (4-block chunks, more only past 4096 items) -> this one: 1
+// sequence of 300 tokens 7.74 -> 6.51, 2000 8.11 -> 7.39, 4200 10.35 -> 9.21,
+// 32768 38.0 -> 27.3; 64 of 300 27.9 -> 19.0; 64 of 1000 59.6 -> 45.5; 8 of
+// 777-6001 33.0 -> 26.3; kvc_decode_attn of 64 of 512-32768 (short chunks,
+// fewer than before) 723 -> 703.
+static int32_t auto_chunk_blocks(const int32_t* nb, int32_t n, bool force_split) {
+    int64_t total = 0;
+    int32_t longest = 1;
+    for (int32_t j = 0; j < n; j++) {
+        total += nb[j];
+        longest = std::max(longest, nb[j]);
+    }
+    // a chunk per sequence needs no exchange: 64 tokens 5.6 us, in two chunks 6.4
+    if (longest <= 3) return 3;
+    // short launches do better with two output-dim parts per chunk than with
+    // twice the chunks: 2 sequences of 1000 tokens 7.6 us against 8.3
+    const int32_t max_chunks = force_split || total <= 64 ? 32 : 64;
+    const auto chunks = [&](int32_t cb) {
+        int64_t c = 0;
+        for (int32_t j = 0; j < n; j++) c += (nb[j] + cb - 1) / cb;
+        return c;
+    };
+    const int32_t short_cb = std::max(4, (int32_t)std::lround(0.25 * std::sqrt((double)total)));
+    if (n > max_chunks) return total <= 64 ? 3 : short_cb;
+    // smallest cb with at most max_chunks chunks (monotone in cb)
+    int32_t lo = std::max<int32_t>((longest + 31) / 32, (int32_t)((total + max_chunks - 1) / max_chunks)), hi = longest;
+    while (lo < hi) {
+        const int32_t mid = (lo + hi) / 2;
+        if (chunks(mid) <= max_chunks)
+            hi = mid;
+        else
+            lo = mid + 1;
+    }
+    return lo - total / 64.0 <= 0.5 * std::sqrt((double)total) ? lo : short_cb;
 }
 
 // Argument block of the decode launch over seqs[i0, i0 + n): work split and
@@ -1121,7 +1152,7 @@ static int build_decode_args(kvc_ctx* c, int32_t layer, const int32_t* seqs, int
     const size_t qrow = (size_t)kQHeads * kHeadDim, kvrow = (size_t)kKvHeads * kHeadDim;
     const size_t osz = out_dtype == KVC_DTYPE_BF16 ? 2 : 4;
     memset(&a, 0, sizeof a);
-    int64_t total_blocks = 0;
+    int32_t nblk[kMaxBatch];
     for (int32_t j = 0; j < n; j++) {
         const Seq& s = c->seqs[seqs[i0 + j]];
         const int32_t L = s.len + s.pending;
@@ -1130,19 +1161,18 @@ static int build_decode_args(kvc_ctx* c, int32_t layer, const int32_t* seqs, int
             return set_err(KVC_ERR_STATE, "sequence %d: fused append needs a reserved token", seqs[i0 + j]);
         a.slot[j] = seqs[i0 + j];
         a.kv_len[j] = L;
-        total_blocks += (L + kBlockTok - 1) / kBlockTok;
+        nblk[j] = (L + kBlockTok - 1) / kBlockTok;
     }
-    int32_t cb = auto_chunk_blocks(c, total_blocks);
     const bool auto_cb = c->cfg.decode_chunk_blocks <= 0;
     const bool force_split = c->cfg.flags & KVC_FLAG_DECODE_SPLIT_D;
+    int32_t cb = auto_cb ? auto_chunk_blocks(nblk, n, force_split) : c->cfg.decode_chunk_blocks;
     const int64_t max_chunks = force_split ? kMaxChunks / kMaxDParts : kMaxChunks;
     int64_t total_chunks;
     for (;;) {
         total_chunks = 0;
         for (int32_t j = 0; j < n; j++) {
             a.chunk_begin[j] = (int32_t)total_chunks;
-            const int32_t nb = (a.kv_len[j] + kBlockTok - 1) / kBlockTok;
-            total_chunks += (nb + cb - 1) / cb;
+            total_chunks += (nblk[j] + cb - 1) / cb;
         }
         // an automatic chunk also grows until the launch has at most
         // kAutoItems items (each sequence's last, partial chunk adds one per
@@ -1153,9 +1183,10 @@ static int build_decode_args(kvc_ctx* c, int32_t layer, const int32_t* seqs, int
         if (total_chunks <= max_chunks && (!auto_cb || auto_items <= kAutoItems)) break;
         cb *= 2;
     }
+    // two output-dim parts per chunk while both still find a CU of their own
     int32_t d_parts = 1;
     if (force_split ||
-        (!(c->cfg.flags & KVC_FLAG_DECODE_NO_SPLIT_D) && total_chunks * kKvHeads < kDsplitBelowItems))
+        (!(c->cfg.flags & KVC_FLAG_DECODE_NO_SPLIT_D) && total_chunks * kKvHeads * kMaxDParts <= 256))
         d_parts = 2;
     const int64_t items = total_chunks * kKvHeads * d_parts;
     if (items > max_items)

@@ -1,0 +1,91 @@
+"""GPU parity of decode's automatic work split at the edges of its rule (one
+chunk per sequence, one workgroup per CU with and without the output-dim
+split, short chunks for very unequal lengths), against the oracle
+(src/engine.cpp:3528-3564): max |diff| <= 2e-2 and relative RMS <= 3e-3; and of
+the one-token Gated-DeltaNet step on either side of its workgroup sizes, bit
+for bit."""
+import numpy as np
+import pytest
+
+import _oracle as O
+import kvc
+from gpu_util import D, NQ, Mirror, fill_seq, say
+
+pytestmark = pytest.mark.gpu
+
+CASES = {
+    "one_chunk": [1, 31, 96],                 # every sequence in one chunk of 3 blocks
+    "four_blocks": [97],                      # first length in several chunks
+    "one_block_chunks": [1024],               # 32 chunks of one block
+    "past_32_chunks": [1025],                 # 33 blocks: chunks of two
+    "short_launch": [1000, 1024],             # 64 blocks: 32 chunks, two parts
+    "past_short_launch": [1000, 1056],        # 65 blocks: chunks of one block, one part
+    "ragged_one_round": [777, 2001, 65, 1500],
+    "very_ragged": [9000] + [33] * 40,        # short chunks
+    "full_batch": [40 + 7 * i for i in range(64)],
+}
+
+
+@pytest.mark.parametrize("flags", [0, kvc.FLAG_DECODE_SPLIT_D, kvc.FLAG_DECODE_NO_SPLIT_D])
+@pytest.mark.parametrize("name", CASES)
+def test_decode_automatic_split(name, flags):
+    lengths = CASES[name]
+    say(f"decode split {name}, flags {flags}")
+    h = kvc.hip()
+    n = len(lengths)
+    with kvc.Context(n_attn_layers=1, n_ssm_layers=0, max_seqs=n, max_seq_len=max(lengths) + 32,
+                     pool_blocks=sum(x // 32 + 1 for x in lengths) + 8, snapshot_slots=0, alloc_seed=77,
+                     flags=flags) as ctx:
+        m = Mirror(1)
+        seqs = [ctx.seq_create() for _ in lengths]
+        for s, x in zip(seqs, lengths):
+            fill_seq(ctx, m, [s], x, seed=500 + x)
+        q = O.normal_bf16(n * NQ * D, 42).reshape(n, NQ * D)
+        qb, ob = kvc.to_device(q), h.malloc(n * NQ * D * 4)
+        ctx.decode_attn(0, seqs, qb, ob)
+        ctx.sync()
+        out = ob.download(np.float32, (n, NQ, D))
+        qb.free()
+        ob.free()
+    for i, x in enumerate(lengths):
+        kk, vv = m.get(seqs[i], 0)
+        O.assert_attn_close(out[i], O.decode_attn(q[i], kk, vv, x), rel_rms=3e-3, what=f"{name}: length {x}")
+
+
+def test_deltanet_one_token_workgroup_sizes():
+    """16 sequences take 1024-thread workgroups, 17 take 512: same bits."""
+    say("deltanet, one token, 16 and 17 sequences")
+    h = kvc.hip()
+    rng = np.random.default_rng(5)
+    C, PROJ, OUT = O.SSM_C, O.SSM_PROJ, O.SSM_NV * O.SSM_DV
+    n = 17
+    w = [(0.5 * rng.standard_normal((4, C))), rng.standard_normal(O.SSM_NV),
+         -rng.uniform(0.05, 1.0, O.SSM_NV), rng.uniform(0.5, 1.5, O.SSM_DV)]
+    proj = O.f32_to_bf16(rng.standard_normal((3, n, PROJ)).astype(np.float32))
+    with kvc.Context(n_attn_layers=1, n_ssm_layers=1, max_seqs=2 * n, max_seq_len=64, pool_blocks=8,
+                     snapshot_slots=0) as ctx:
+        bufs = [kvc.to_device(x.astype(np.float32)) for x in w]
+        sets = [[ctx.seq_create() for _ in range(n)] for _ in range(2)]
+        got = []
+        for group, parts in zip(sets, ((n,), (16, 1))):
+            outs = []
+            for step in range(3):
+                pb, ob = kvc.to_device(proj[step]), h.malloc(n * OUT * 4)
+                i0 = 0
+                for k in parts:
+                    ctx.deltanet_step(0, group[i0:i0 + k], 1, pb.ptr + i0 * PROJ * 2, *bufs, ob.ptr + i0 * OUT * 4)
+                    i0 += k
+                ctx.sync()
+                outs.append(ob.download(np.float32, (n, OUT)))
+                pb.free()
+                ob.free()
+            state = []
+            for s in group:
+                r, c = ctx.state_ptrs(s, 0)
+                state.append(kvc.DeviceBuffer(h, r, OUT * O.SSM_DK * 4).download(np.uint32, (OUT * O.SSM_DK,)))
+                state.append(kvc.DeviceBuffer(h, c, 3 * C * 4).download(np.uint32, (3 * C,)))
+            got.append((outs, state))
+        for b in bufs:
+            b.free()
+    for a, b in zip(got[0][0] + got[0][1], got[1][0] + got[1][1]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
