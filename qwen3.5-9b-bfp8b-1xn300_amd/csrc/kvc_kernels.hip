@@ -1419,7 +1419,7 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
 // other's LDS reads and softmax, and each K/V tile serves 32 rows.  ROWS = 16
 // (4 waves, one per SIMD) is for launches that leave CUs idle anyway: half the
 // rows per workgroup halves its q arithmetic, softmax and gate epilogue, which
-// share the SIMDs' VALUs (prefill_rows in the host code has the rule).
+// share the SIMDs' VALUs (prefill_split in the host code has the rule).
 //
 // The per-tile VALU work is kept small:
 //  - tiles are fetched with the scalar-base form of the LDS DMA, with
@@ -1446,7 +1446,7 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
 // block's keys and leaves its unnormalised output and row statistics in the
 // workspace for prefill_combine_kernel; a block that one piece covers is
 // finished here.  Chosen by the host for launches that would leave most CUs
-// idle (prefill_piece_tiles).
+// idle (prefill_split).
 template <int ROWS, int PROD, bool SPLIT>
 // (launch bounds of 512 threads in either size: told of 256, the compiler
 // plans for one wave per SIMD and keeps the accumulators in AGPRs, which cost
@@ -3241,8 +3241,8 @@ void deltanet_mfma_kernel(DeltaNetArgs a) {
 // Rows of Wk are beta_t e^{g_t} k_t^T times a product of (I - beta k k^T), so
 // their entries stay below beta_t e^{g_t}: a power of two from that bound is
 // the row's scale for the two-part fp16 split (the other splits as above).
-// 500 tokens of one sequence: 206.6 -> 58.0 us per layer (front 15.4, state 35.9,
-// norm 6.8); the errors against a 64-bit result are no larger than the
+// 500 tokens of one sequence: 206.6 -> 56.4 us per layer (front 15.1, state 35.0,
+// norm 6.1); the errors against a 64-bit result are no larger than the
 // persistent kernel's (fp32 outputs 2.5e-7 against 2.6e-7).
 //
 // Workspace of one (sequence, k-head, block), in 16-B pieces: Q's split
@@ -3706,48 +3706,45 @@ void deltanet_state_kernel(DeltaNetArgs a) {
     }
 }
 
-// Gated RMSNorm of O: one wave per (sequence, k-head, block, v-head); lane
-// (g, c) holds tokens 4 r + g of columns 16 vt + c.
+// Gated RMSNorm of O: one workgroup per (sequence, k-head, block, v-head), wave
+// r taking tokens 4 r + g: lane (g, c) holds columns 16 vt + c of its token.
+// Bounded by the latency of its loads and stores: a wave with all 16 tokens
+// issues 40 loads and 32 stores, 16 and 8 here.  500 tokens of one sequence 7.30
+// -> 6.08 us.
 template <bool BF16IN, bool REF>
 __global__ __launch_bounds__(256) void deltanet_norm_kernel(DeltaNetArgs a) {
 #pragma clang fp contract(off)
-    const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    const int h = w & 1, ib = w >> 1;
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = blockIdx.x & 1, ib = blockIdx.x >> 1;
     const int item = ib / a.seg_blocks, blk = ib % a.seg_blocks + a.seg_begin;
     const int seq = item / kSsmKHeads, vh = item % kSsmKHeads + kSsmKHeads * h;
-    const f32x4* src = reinterpret_cast<const f32x4*>(a.ws) + (size_t)ib * kDfSize + kDfHead + h * kDfHeadSize + kDfUv + lane;
-    const int tok0 = blk * kDnChunk + g;
-    size_t zrow[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-        zrow[r] = ((size_t)seq * a.n_tok + min(tok0 + 4 * r, a.n_tok - 1)) * kSsmProj + kSsmC + (size_t)vh * kSsmDv + c;
-    f32x4 o[8];
-    uint32_t z[8][4];
-    float nw[8];
+    const int tok = blk * kDnChunk + 4 * r + g;
+    if (tok - g >= a.n_tok) return;
+    const float* src = reinterpret_cast<const float*>(reinterpret_cast<const u32x4*>(a.ws) + (size_t)ib * kDfSize + kDfHead +
+                                                      h * kDfHeadSize + kDfUv + lane) + r;
+    const size_t zrow = ((size_t)seq * a.n_tok + min(tok, a.n_tok - 1)) * kSsmProj + kSsmC + (size_t)vh * kSsmDv + c;
+    float o[8], nw[8];
+    uint32_t z[8];
 #pragma unroll
     for (int vt = 0; vt < 8; vt++) {
-        o[vt] = src[vt * 64];
+        o[vt] = src[vt * 256];
+        z[vt] = load_raw<BF16IN>(a.proj, zrow + 16 * vt);
         nw[vt] = a.norm_w[16 * vt + c];
-#pragma unroll
-        for (int r = 0; r < 4; r++) z[vt][r] = load_raw<BF16IN>(a.proj, zrow[r] + 16 * vt);
     }
+    float ss = 0.f;
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        float ss = 0.f;
+    for (int vt = 0; vt < 8; vt++) ss = fmaf(o[vt], o[vt], ss);
+    const float rms = dn_rsqrt(sum16(ss) / kSsmDv + a.eps);
+    if (tok >= a.n_tok) return;
+    const size_t oi = ((size_t)seq * a.n_tok + tok) * (kSsmVHeads * kSsmDv) + (size_t)vh * kSsmDv + c;
 #pragma unroll
-        for (int vt = 0; vt < 8; vt++) ss = fmaf(o[vt][r], o[vt][r], ss);
-        const float rms = dn_rsqrt(sum16(ss) / kSsmDv + a.eps);
-        const int tok = tok0 + 4 * r;
-        if (tok >= a.n_tok) continue;
-        const size_t oi = ((size_t)seq * a.n_tok + tok) * (kSsmVHeads * kSsmDv) + (size_t)vh * kSsmDv + c;
-#pragma unroll
-        for (int vt = 0; vt < 8; vt++) {
-            const float y = o[vt][r] * rms * nw[vt] * dn_silu<REF>(raw_f<BF16IN>(z[vt][r]));
-            if (a.out_bf16)
-                static_cast<uint16_t*>(a.out)[oi + 16 * vt] = (uint16_t)f32_to_bf16_rne(y);
-            else
-                static_cast<float*>(a.out)[oi + 16 * vt] = y;
-        }
+    for (int vt = 0; vt < 8; vt++) {
+        const float y = o[vt] * rms * nw[vt] * dn_silu<REF>(raw_f<BF16IN>(z[vt]));
+        if (a.out_bf16)
+            static_cast<uint16_t*>(a.out)[oi + 16 * vt] = (uint16_t)f32_to_bf16_rne(y);
+        else
+            static_cast<float*>(a.out)[oi + 16 * vt] = y;
     }
 }
 
@@ -4208,7 +4205,7 @@ static void launch_deltanet_t(const DeltaNetArgs& a, hipStream_t stream) {
             d.seg_begin = b;
             d.seg_blocks = std::min(a.seg_blocks, nblk - b);
             d.seg_last = b + d.seg_blocks == nblk;
-            const dim3 fgrid(items * d.seg_blocks), sgrid(a.n_seqs * kSsmVHeads * 2), ngrid(items * d.seg_blocks / 2);
+            const dim3 fgrid(items * d.seg_blocks), sgrid(a.n_seqs * kSsmVHeads * 2), ngrid(items * d.seg_blocks * 2);
             if (a.in_bf16) {
                 hipLaunchKernelGGL((deltanet_front_kernel<true, REF>), fgrid, dim3(kDfThreads), 0, stream, d);
                 hipLaunchKernelGGL((deltanet_state_kernel<true>), sgrid, dim3(kDfStateThreads), 0, stream, d);
