@@ -1579,7 +1579,7 @@ int kvc_state_ptrs(kvc_ctx* c, int32_t seq, int32_t ssm_layer, void** rec, void*
 // at a time; the other kernels run 16 per sequence, token by token up to 12
 // tokens and in 6 us per 16-token block from 13.  us per layer, other kernel /
 // few-sequence form: 1 sequence, 8 tokens 15.8 / 17.5, 9 tokens 20.1 / 18.1,
-// 128 tokens 64.2 / 30.6, 500 tokens 206.6 / 58.0; 4 sequences, 9 tokens 20.9 /
+// 128 tokens 64.2 / 30.6, 500 tokens 206.6 / 56.4; 4 sequences, 9 tokens 20.9 /
 // 21.1, 12 tokens 24.6 / 21.6, 512 tokens 210 / 93; 5 sequences, 32 tokens
 // 29.5 / 30.0, 48 tokens 35.5 / 33.7; 7 sequences, 64 tokens 42.0 / 42.8, 96
 // tokens 54.8 / 53.2; 8 sequences, 512 tokens 210.5 / 206.9; 10 sequences 211.5

@@ -1,7 +1,8 @@
 """GPU parity of decode's automatic work split at the edges of its rule (one
 chunk per sequence, one workgroup per CU with and without the output-dim
 split, short chunks for very unequal lengths), against the oracle
-(src/engine.cpp:3528-3564): max |diff| <= 2e-2 and relative RMS <= 3e-3; and of
+(src/engine.cpp:3528-3564): max |diff| <= 2e-2 and relative RMS <= 3e-3; of its
+weight offset under scores that move by hundreds of bits, with the same bars; and of
 the one-token Gated-DeltaNet step on either side of its workgroup sizes, bit
 for bit."""
 import numpy as np
@@ -9,7 +10,7 @@ import pytest
 
 import _oracle as O
 import kvc
-from gpu_util import D, NQ, Mirror, fill_seq, say
+from gpu_util import D, NKV, NQ, Mirror, fill_seq, say
 
 pytestmark = pytest.mark.gpu
 
@@ -50,6 +51,45 @@ def test_decode_automatic_split(name, flags):
     for i, x in enumerate(lengths):
         kk, vv = m.get(seqs[i], 0)
         O.assert_attn_close(out[i], O.decode_attn(q[i], kk, vv, x), rel_rms=3e-3, what=f"{name}: length {x}")
+
+
+# mean score of each group of 4 blocks, in units of 23 bits of the weights: the
+# walk moves its weight offset at each group's first block, downwards by 16
+# bits of the largest score at most
+LEVELS = {
+    "falling": [-2.0 * i for i in range(12)],   # 500 bits in all: an unbounded offset overflows
+    "falling_slowly": [-0.3 * i for i in range(12)],
+    "rising": [2.0 * i for i in range(12)],
+    "alternating": [0.0, -0.5, 0.1, -3.0, 0.2, -0.6] * 2,
+    "late_peak": [-4.0] * 11 + [0.0],
+}
+
+
+@pytest.mark.parametrize("flags", [kvc.FLAG_DECODE_SPLIT_D, kvc.FLAG_DECODE_NO_SPLIT_D])
+@pytest.mark.parametrize("name", LEVELS)
+def test_decode_weight_offset(name, flags):
+    say(f"decode weight offset {name}, flags {flags}")
+    h = kvc.hip()
+    L = 12 * 128 - 27
+    rng = np.random.default_rng(9)
+    lev = np.repeat(np.asarray(LEVELS[name], np.float32), 128)[:L, None]
+    k = O.f32_to_bf16(lev + 0.1 * rng.standard_normal((L, NKV * D)).astype(np.float32))
+    v = O.normal_bf16(L * NKV * D, 91).reshape(L, NKV * D)
+    q = O.f32_to_bf16(np.ones(NQ * D, np.float32))
+    with kvc.Context(n_attn_layers=1, n_ssm_layers=0, max_seqs=1, max_seq_len=L + 32, pool_blocks=L // 32 + 8,
+                     snapshot_slots=0, alloc_seed=78, decode_chunk_blocks=48, flags=flags) as ctx:
+        s = ctx.seq_create()
+        ctx.reserve([s], L)
+        bufs = [kvc.to_device(x) for x in (k, v, q)]
+        ob = h.malloc(NQ * D * 4)
+        ctx.append(0, [s], L, bufs[0], bufs[1])
+        ctx.commit([s], L)
+        ctx.decode_attn(0, [s], bufs[2], ob)
+        ctx.sync()
+        out = ob.download(np.float32, (NQ, D))
+        for b in bufs + [ob]:
+            b.free()
+    O.assert_attn_close(out, O.decode_attn(q, k, v, L), rel_rms=3e-3, what=name)
 
 
 def test_deltanet_one_token_workgroup_sizes():
