@@ -252,7 +252,7 @@ struct PrefillArgs {
     int32_t gate_ref;           // 1: the reference's Schraudolph gate sigmoid; 0: exact
     int32_t n_groups;           // n_seqs * Hkv (sequence, kv head) groups
     int32_t pad2;
-    // prefill with the producer's q side fused in (prefill_mfma_kernel<NT, 1 or 2>):
+    // prefill with the producer's q side fused in (prefill_mfma_kernel<ROWS, 1 or 2, SPLIT>):
     // q and gate come from the projection rows
     const void* qkv;            // [n_seqs][n_q][kQkvRow] (layout of QkvArgs::qkv), bf16 or fp32
     const float* q_norm;        // [D]
