@@ -15,7 +15,7 @@ constexpr int kWaves = 4;           // waves per decode workgroup (each takes 8 
 constexpr int kTokPerWave = kBlockTok / kWaves;  // 8 tokens of a block per wave
 constexpr float kNegBig = -1.0e30f;
 constexpr float kRescaleSlack = 8.0f;  // lazy rescale: p may reach 2^8
-constexpr float kRescaleDrop = 16.0f;  // the offset stays within 2^16 of the largest score met
+constexpr float kRescaleDrop = 16.0f;  // the offset falls at most 16 bits below its highest so far
 
 // ---------------------------------------------------------------------------
 // Block-table update: entries ride in the argument block.
@@ -30,8 +30,8 @@ __global__ void table_update_kernel(TableUpdateArgs a) {
 struct WaveState {
     float m[kGroup];  // filled by finalize_l
     float l[kGroup];
-    // of the lane's head: weight offset (weights are 2^(score - m)), largest
-    // score of the groups' first blocks, and the lane's part of the denominator
+    // of the lane's head: weight offset (weights are 2^(score - m)), the highest
+    // that the offset has been, and the lane's part of the denominator
     float m_lane, top, l_lane;
     float acc[kGroup][4];
 };
@@ -130,13 +130,17 @@ __device__ __forceinline__ float bf16_round(float x) { return __uint_as_float(cv
 // qv[g][j][i]: packed bf16 pairs of q head g, dims (c + 16j)*8 + 2i, +1.
 // lds_p16: per-wave 32 bf16 p values laid out [g][token].
 // FIRST (the first block of a group of 4): the offset moves to the block's
-// largest score, whose weight is then 1 and exact in bf16, also downwards (as
-// far as kRescaleDrop allows).  Heavy weights carry most of the rounding
+// largest score, whose weight is then 1 and exact in bf16, also downwards, but
+// not further than kRescaleDrop below its highest so far (top, which every rise
+// updates).  A score is at most the offset plus the slack where it is met, so
+// no weight already summed exceeds 2^(kRescaleDrop + kRescaleSlack) and no
+// rescale factor 2^kRescaleDrop.  Heavy weights carry most of the rounding
 // error: 8 sequences of 777-6001 tokens in long chunks, fp32 out, are 1.61e-3
 // off the 64-bit result with an offset that only rises past the slack and
 // 1.46e-3 with this one.  Each lane keeps its head's offset, 3 or 4 VGPRs
-// less than four wave-uniform copies and their selects.  Both, us per layer: 1 sequence of 300 tokens 6.60 -> 6.44, of 4096 8.51 ->
-// 8.40, the 8 sequences 26.4 -> 26.5, 64 of 512-32768 702.6 -> 701.1.
+// less than four wave-uniform copies and their selects.  Both, us per layer: 1
+// sequence of 300 tokens 6.60 -> 6.44, of 4096 8.51 -> 8.40, the 8 sequences
+// 26.4 -> 26.5, 64 of 512-32768 702.6 -> 701.1.
 template <int NP, bool FIRST>
 __device__ __forceinline__ void compute_block(BlockRegs<NP>& r, const uint32_t (&qv)[kGroup][2][4],
                                               int n_valid, float scale_log2, uint16_t* lds_p16,
@@ -191,12 +195,11 @@ __device__ __forceinline__ void compute_block(BlockRegs<NP>& r, const uint32_t (
         mx = fmaxf(mx, dpp<kDppRowRor8>(mx));
         mx = max_xor16(mx);
         mx = max_xor32(mx);
-        if constexpr (FIRST) {
-            st.top = fmaxf(st.top, mx);
+        if constexpr (FIRST)
             mx = fmaxf(mx, st.top - kRescaleDrop);
-        } else {
+        else
             mx = mx > st.m_lane + kRescaleSlack ? mx : st.m_lane;
-        }
+        st.top = fmaxf(st.top, mx);
         const float c_own = fast_exp2(st.m_lane - mx);
         st.m_lane = mx;
         st.l_lane *= c_own;

@@ -2,7 +2,8 @@
 chunk per sequence, one workgroup per CU with and without the output-dim
 split, short chunks for very unequal lengths), against the oracle
 (src/engine.cpp:3528-3564): max |diff| <= 2e-2 and relative RMS <= 3e-3; of its
-weight offset under scores that move by hundreds of bits, with the same bars; and of
+weight offset under scores that move by hundreds of bits from group to group or
+by one key in any block of a group, with the same bars; and of
 the one-token Gated-DeltaNet step on either side of its workgroup sizes, bit
 for bit."""
 import numpy as np
@@ -90,6 +91,41 @@ def test_decode_weight_offset(name, flags):
         for b in bufs + [ob]:
             b.free()
     O.assert_attn_close(out, O.decode_attn(q, k, v, L), rel_rms=3e-3, what=name)
+
+
+@pytest.mark.parametrize("flags", [kvc.FLAG_DECODE_SPLIT_D, kvc.FLAG_DECODE_NO_SPLIT_D])
+@pytest.mark.parametrize("bits", [100, 150, 500])
+@pytest.mark.parametrize("block", range(8))
+def test_decode_weight_offset_single_peak(block, bits, flags):
+    """One key `bits` bits above all others, in each block of a group of 4 (the
+    offset moves down only at a group's first), followed by lower groups and a
+    tail of 3 blocks, and in each wave's 8 tokens of the block: the largest
+    score met has to bound the offset wherever it stood."""
+    say(f"decode weight offset, peak of {bits} bits in block {block}, flags {flags}")
+    h = kvc.hip()
+    L = 11 * 32 - 5
+    rng = np.random.default_rng(10 + block)
+    lev = np.zeros((L, 1), np.float32)
+    wave = (block + bits // 50) % 4
+    lev[32 * block + 8 * wave + block % 8] = bits / 23.08
+    k = O.f32_to_bf16(lev + 0.1 * rng.standard_normal((L, NKV * D)).astype(np.float32))
+    v = O.normal_bf16(L * NKV * D, 92 + block).reshape(L, NKV * D)
+    q = O.f32_to_bf16(np.ones(NQ * D, np.float32))
+    with kvc.Context(n_attn_layers=1, n_ssm_layers=0, max_seqs=1, max_seq_len=L + 32, pool_blocks=L // 32 + 8,
+                     snapshot_slots=0, alloc_seed=79, decode_chunk_blocks=16, flags=flags) as ctx:
+        s = ctx.seq_create()
+        ctx.reserve([s], L)
+        bufs = [kvc.to_device(x) for x in (k, v, q)]
+        ob = h.malloc(NQ * D * 4)
+        ctx.append(0, [s], L, bufs[0], bufs[1])
+        ctx.commit([s], L)
+        ctx.decode_attn(0, [s], bufs[2], ob)
+        ctx.sync()
+        out = ob.download(np.float32, (NQ, D))
+        for b in bufs + [ob]:
+            b.free()
+    assert np.isfinite(out).all()
+    O.assert_attn_close(out, O.decode_attn(q, k, v, L), rel_rms=3e-3, what=f"peak in block {block}")
 
 
 def test_deltanet_one_token_workgroup_sizes():
