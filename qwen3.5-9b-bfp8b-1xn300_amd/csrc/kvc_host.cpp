@@ -1574,18 +1574,21 @@ int kvc_state_ptrs(kvc_ctx* c, int32_t seq, int32_t ssm_layer, void** rec, void*
     return KVC_OK;
 }
 
-// Whether a launch takes the few-sequence matrix form.  Its three launches cost
-// more than one, and its state pass runs 64 workgroups per sequence, one per CU
-// at a time; the other kernels run 16 per sequence, token by token up to 12
-// tokens and in 6 us per 16-token block from 13.  us per layer, other kernel /
-// few-sequence form: 1 sequence, 8 tokens 15.8 / 17.5, 9 tokens 20.1 / 18.1,
-// 128 tokens 64.2 / 30.6, 500 tokens 206.6 / 56.4; 4 sequences, 9 tokens 20.9 /
-// 21.1, 12 tokens 24.6 / 21.6, 512 tokens 210 / 93; 5 sequences, 32 tokens
-// 29.5 / 30.0, 48 tokens 35.5 / 33.7; 7 sequences, 64 tokens 42.0 / 42.8, 96
-// tokens 54.8 / 53.2; 8 sequences, 512 tokens 210.5 / 206.9; 10 sequences 211.5
-// / 268.2.
+// Whether a launch takes the few-sequence matrix form: where calls of more
+// sequences run a matrix form too (up to 12 tokens the kernels hold everything
+// in fp32 and give the bits of one-token steps, which this form's two-part
+// splits do not: state 1.1-1.8 times as far from a 64-bit result at 9-12
+// tokens, 10 times with large inputs), and where it is the faster one.  Its
+// three launches cost more than one, and its state pass runs 64 workgroups per
+// sequence, one per CU at a time; the persistent kernel runs 16 per sequence,
+// in 6 us per 16-token block.  us per layer, persistent kernel / few-sequence
+// form: 1 sequence, 13 tokens 21.6 / 16.2, 128 tokens 64.2 / 30.6, 500 tokens
+// 206.6 / 56.4; 4 sequences, 13 tokens 22.9 / 19.6, 512 tokens 210 / 93; 5
+// sequences, 32 tokens 29.5 / 30.0, 48 tokens 35.5 / 33.7; 7 sequences, 64
+// tokens 42.0 / 42.8, 96 tokens 54.8 / 53.2; 8 sequences, 512 tokens 210.5 /
+// 206.9; 10 sequences 211.5 / 268.2.
 static bool deltanet_few(int32_t n_seqs, int32_t n_tok) {
-    if (n_seqs <= 4) return n_tok >= (n_seqs < 4 ? 9 : 10);
+    if (n_seqs <= 4) return n_tok >= kSsmMatrixMin;
     return n_seqs <= 7 && n_tok > kSsmChunk * (n_seqs - 3);
 }
 

@@ -194,6 +194,7 @@ struct DeltaNetArgs {
     int32_t slot[kMaxBatch];
 };
 constexpr int kSsmChunk = 16;       // tokens per block of the matrix forms
+constexpr int kSsmMatrixMin = 13;   // fewest tokens of a call that runs one (kvc_kernels.hip)
 constexpr int kDnFewBytes = 53248;
 constexpr int kDnFewMax = (int)(kPartBytes / kDnFewBytes);
 

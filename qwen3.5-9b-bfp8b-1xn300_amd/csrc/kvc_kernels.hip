@@ -2563,7 +2563,7 @@ constexpr int kDnChunk = kSsmChunk;
 // below 16).  Measured at config e (64 sessions, interleaved): the blocked
 // kernel takes 84.0-85.4 / 89.9-90.2 us per layer at 12 / 13 tokens, the
 // matrix form 86.8 / 86.9-87.1; the two meet between 12 and 13.
-constexpr int kDnMatrixMin = 13;
+constexpr int kDnMatrixMin = kSsmMatrixMin;
 static_assert(kDnMatrixMin <= 2 * kDnBlk, "the blocked kernel covers calls of at most two blocks");
 
 __device__ __forceinline__ int dn_sigma(int r) { return 4 * (r & 3) + (r >> 2); }

@@ -6,17 +6,18 @@ few-sequence form.  The oracle and the fp32 bars are those files'."""
 import numpy as np
 import pytest
 
+import _oracle as O
 import kvc
 from gpu_util import say
-from test_gpu_deltanet import run_case
+from test_gpu_deltanet import ctx_ssm, run_case, state_bufs
 from test_gpu_deltanet_ranges import check_all, run
 
 pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n_tok,n_seqs,in_dtype,out_dtype", [
-    (9, 1, kvc.DTYPE_BF16, kvc.DTYPE_F32),    # shortest: one block of 9
-    (10, 4, kvc.DTYPE_F32, kvc.DTYPE_F32),    # shortest of 4 sequences
+    (13, 1, kvc.DTYPE_BF16, kvc.DTYPE_F32),   # shortest: one block of 13
+    (13, 4, kvc.DTYPE_F32, kvc.DTYPE_F32),    # shortest of 4 sequences
     (16, 1, kvc.DTYPE_BF16, kvc.DTYPE_BF16),  # one whole block
     (17, 3, kvc.DTYPE_F32, kvc.DTYPE_BF16),   # a second block of one token
     (95, 2, kvc.DTYPE_BF16, kvc.DTYPE_F32),   # more blocks than LDS buffers, ragged end
@@ -27,6 +28,42 @@ pytestmark = pytest.mark.gpu
 def test_few_sequences(n_tok, n_seqs, in_dtype, out_dtype):
     say(f"deltanet, {n_seqs} sequences of {n_tok} tokens, in {in_dtype} out {out_dtype}")
     run_case(in_dtype, out_dtype, n_tok=n_tok, n_seqs=n_seqs, seed=12000 + 7 * n_tok + n_seqs)
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("n_seqs", [1, 2, 3, 4])
+@pytest.mark.parametrize("n_tok", [2, 8, 9, 10, 11, 12])
+def test_short_calls_have_the_bits_of_token_steps(n_tok, n_seqs, exact):
+    """Up to 12 tokens, however few the sequences, the arithmetic is fp32
+    throughout and the same as token by token: outputs and state bit for bit."""
+    say(f"deltanet, {n_seqs} sequences of {n_tok} tokens against token steps, exact {exact}")
+    h = kvc.hip()
+    rng = np.random.default_rng(12500 + 10 * n_tok + n_seqs)
+    OUT = O.SSM_NV * O.SSM_DV
+    w = [0.5 * rng.standard_normal((4, O.SSM_C)), rng.standard_normal(O.SSM_NV), -rng.uniform(0.05, 1.0, O.SSM_NV),
+         rng.uniform(0.5, 1.5, O.SSM_DV)]
+    proj = O.f32_to_bf16(rng.standard_normal((n_seqs, n_tok, O.SSM_PROJ)).astype(np.float32))
+    S0 = (0.05 * rng.standard_normal(OUT * O.SSM_DK)).astype(np.float32)
+    got = []
+    with ctx_ssm(max_seqs=2 * n_seqs, flags=kvc.FLAG_EXACT_MATH if exact else 0) as ctx:
+        bufs = [kvc.to_device(x.astype(np.float32)) for x in w]
+        for step in (n_tok, 1):
+            seqs = [ctx.seq_create() for _ in range(n_seqs)]
+            for s in seqs:
+                state_bufs(ctx, s, 0)[0].upload(S0)
+            out = np.empty((n_seqs, n_tok, OUT), np.float32)
+            for t in range(0, n_tok, step):
+                pb, ob = kvc.to_device(np.ascontiguousarray(proj[:, t:t + step])), h.malloc(n_seqs * step * OUT * 4)
+                ctx.deltanet_step(0, seqs, step, pb, *bufs, ob)
+                ctx.sync()
+                out[:, t:t + step] = ob.download(np.float32, (n_seqs, step, OUT))
+                pb.free()
+                ob.free()
+            got.append([out] + [b.download(np.float32, (b.nbytes // 4,)) for s in seqs for b in state_bufs(ctx, s, 0)])
+        for b in bufs:
+            b.free()
+    for a, b in zip(*got):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
 def test_few_sequences_over_workspace_segments():
