@@ -25,6 +25,7 @@
 
 #include "../../include/kvc.h"
 #include "kvc_internal.h"
+#include "kvc_prefill_split.h"
 
 using namespace kvc;
 
@@ -1294,66 +1295,6 @@ int kvc_decode_attn_static(kvc_ctx* c, int32_t layer, const int32_t* seqs, int32
     return decode_impl(c, layer, seqs, n_seqs, q, k_new, v_new, gate, DecodeProducer{}, out, out_dtype, scale,
                        stream, c ? c->s_part : nullptr, (uint32_t)kStaticPartBytes, c ? c->s_counters : nullptr,
                        kStaticItems, "static decode workspace");
-}
-
-// Work split of a prefill launch: rows per workgroup (16 or 32) and key tiles
-// per piece (0: groups are not split).  One workgroup runs per CU, so a launch
-// of few workgroups, or of workgroups of very unequal lengths, takes as long as
-// its longest one; 16-row workgroups are shorter, and cut into pieces a launch
-// takes as long as its work spread over all CUs plus the fold of the pieces.
-// Each choice is priced (us, fitted to one MI355X) and the cheapest taken: a
-// workgroup's fixed part (q, first tile, epilogue) and a tile in either size,
-// the fold's launch, a partial written and read at 6 TB/s, and a margin for
-// the split, whose pieces slow each other once they fill the card (64
-// sequences of 8 rows over 100-3000 keys: 116 us unsplit, 129 split).
-// kvc_prefill_step, us per layer, unsplit 32-row workgroups against the
-// choice made: 32 rows over 4001 keys 132.6 -> 27.8; 128 rows over 16000 keys
-// 489 -> 59; 128 rows over 1000 keys 47.2 -> 26.8; 500 rows over none 33.6 ->
-// 28.7 (16 rows, unsplit); 40 sequences of 16 rows over 100-12000 keys 368 ->
-// 237.  Launches of 512 and more 32-row workgroups have no idle CU to fill.
-static void prefill_split(PrefillArgs& a) {
-    constexpr double kCus = 256, kFold = 6.0, kPartBytesPerUs = 6e6, kMargin = 1.15;
-    const auto blocks_of = [&](int rows) { return (a.n_q + rows - 1) / (int64_t)rows; };
-    a.rows = 32;
-    a.piece_tiles = 0;
-    if (a.n_groups * blocks_of(32) >= 2 * (int64_t)kCus) {
-        if (a.n_q <= 16) a.rows = 16;
-        return;
-    }
-    double best = 1e30;
-    for (int rows = 16; rows <= 32; rows += 16) {
-        const double fixed = rows == 16 ? 5.0 : 9.0, tile = rows == 16 ? 1.7 : 1.95;
-        const int64_t n_pb = blocks_of(rows);
-        const auto tiles_of = [&](int32_t j, int64_t b) {
-            return (a.q_pos0[j] + std::min<int64_t>((b + 1) * rows, a.n_q) + kPfKeys - 1) / kPfKeys;
-        };
-        int64_t total = 0, longest = 0;
-        for (int32_t j = 0; j < a.n_seqs; j++)
-            for (int64_t b = 0; b < n_pb; b++) {
-                total += tiles_of(j, b) * kKvHeads;
-                longest = std::max(longest, tiles_of(j, b));
-            }
-        for (int64_t t = longest; t >= 1; t -= std::max<int64_t>(1, t / 5)) {
-            int64_t wgs = 0, parts = 0, slots = 0;
-            for (int32_t j = 0; j < a.n_seqs; j++) {
-                slots += (tiles_of(j, n_pb - 1) + t - 1) / t * kKvHeads * n_pb;
-                for (int64_t b = 0; b < n_pb; b++) {
-                    const int64_t p = (tiles_of(j, b) + t - 1) / t * kKvHeads;
-                    wgs += p;
-                    if (p > kKvHeads) parts += p;
-                }
-            }
-            if (t < longest && slots > pf_max_parts(rows)) break;
-            const double rounds = std::max(1.0, wgs / kCus);
-            double cost = rounds * fixed + tile * (wgs <= kCus ? t : std::max((double)t, total / kCus + 0.5 * t));
-            if (t < longest) cost = kMargin * (cost + kFold + parts * pf_part_floats(rows) * 8 / kPartBytesPerUs);
-            if (cost < best) {
-                best = cost;
-                a.rows = rows;
-                a.piece_tiles = t < longest ? (int32_t)t : 0;
-            }
-        }
-    }
 }
 
 // Prefill launches over all seqs, 64 per launch (arguments checked by the

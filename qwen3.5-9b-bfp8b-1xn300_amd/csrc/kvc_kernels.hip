@@ -1436,7 +1436,7 @@ __device__ __forceinline__ void prefill_q_row(const void* qkv, size_t row, const
 // other's LDS reads and softmax, and each K/V tile serves 32 rows.  ROWS = 16
 // (4 waves, one per SIMD) is for launches that leave CUs idle anyway: half the
 // rows per workgroup halves its q arithmetic, softmax and gate epilogue, which
-// share the SIMDs' VALUs (prefill_split in the host code has the rule).
+// share the SIMDs' VALUs (prefill_split in kvc_prefill_split.h has the rule).
 //
 // The per-tile VALU work is kept small:
 //  - tiles are fetched with the scalar-base form of the LDS DMA, with
