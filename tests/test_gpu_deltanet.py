@@ -267,11 +267,11 @@ def test_deltanet_state_is_zero_after_create_and_reset():
 
 @pytest.mark.parametrize("n_tok", [14, 16, 37, 128])
 def test_deltanet_matrix_form_chunks_match_oracle(n_tok):
-    """Calls of 14 or more tokens take the matrix (WY) form over 16-token
-    blocks on fp32 MFMA; 14 tokens are one partial block and 37 tokens end
-    in one.  Every token's
-    output and the final state are held to the same fp32 bar as the
-    token-by-token kernels."""
+    """Calls of 13 or more tokens take the matrix (WY) form over 16-token
+    blocks on MFMA, of 2 sequences in three launches; 14 tokens are one partial
+    block and 37 tokens end in one.  Every token's output and the final state
+    are held to the same fp32 bar as the token-by-token kernels.  More
+    sequences: test_gpu_deltanet_few.py."""
     say(f"deltanet matrix form, {n_tok} tokens")
     run_case(kvc.DTYPE_BF16, kvc.DTYPE_F32, n_tok=n_tok, n_seqs=2, seed=7700 + n_tok)
 
@@ -356,8 +356,8 @@ def test_deltanet_rejects_rows_past_2gib(in_dtype, n_tok):
 @pytest.mark.parametrize("n_tok", [1, 5, 37])
 def test_deltanet_exact_math_flag_matches_exact_oracle(n_tok):
     """KVC_FLAG_EXACT_MATH: hardware exp / log / reciprocal instead of the
-    reference's Schraudolph forms, through all three kernels (1 token, the
-    blocked kernel, the matrix form), against the oracle's fast = 0."""
+    reference's Schraudolph forms, through the one-token and the blocked kernel
+    and the few-sequence matrix form, against the oracle's fast = 0."""
     say(f"deltanet exact-math flag, {n_tok} tokens")
     run_case(kvc.DTYPE_BF16, kvc.DTYPE_F32, n_tok=n_tok, n_seqs=2, seed=8100 + n_tok, exact=True)
 

@@ -1,8 +1,10 @@
 """GPU parity of the Gated-DeltaNet matrix form for few sequences (front, state
 and norm launches; src/engine.cpp:2600-2716) at the edges of its blocks,
-sequence counts and workspace segments, and of the persistent matrix form at
-the ranges that test_gpu_deltanet_ranges.py now reaches only through the
-few-sequence form.  The oracle and the fp32 bars are those files'."""
+sequence counts and workspace segments; of the kernels that calls of more
+sequences run, in the types, math modes and ranges that test_gpu_deltanet.py and
+test_gpu_deltanet_ranges.py, with few sequences, reach only through other
+kernels; and of short calls against one-token steps, bit for bit.  The oracle
+and the fp32 bars are those files'."""
 import numpy as np
 import pytest
 
@@ -71,6 +73,34 @@ def test_few_sequences_over_workspace_segments():
     so the call runs as two segments of blocks."""
     say("deltanet, 4 sequences of 700 tokens in two workspace segments")
     run_case(kvc.DTYPE_BF16, kvc.DTYPE_F32, n_tok=700, n_seqs=4, seed=12900)
+
+
+@pytest.mark.parametrize("n_tok,n_seqs,in_dtype,out_dtype,exact", [
+    # the persistent matrix form: every type and math mode
+    (16, 8, kvc.DTYPE_BF16, kvc.DTYPE_BF16, False),
+    (33, 8, kvc.DTYPE_BF16, kvc.DTYPE_BF16, True),
+    (37, 8, kvc.DTYPE_BF16, kvc.DTYPE_F32, True),
+    (20, 9, kvc.DTYPE_F32, kvc.DTYPE_BF16, False),
+    (37, 8, kvc.DTYPE_F32, kvc.DTYPE_BF16, True),
+    (17, 8, kvc.DTYPE_F32, kvc.DTYPE_F32, True),
+    (13, 5, kvc.DTYPE_F32, kvc.DTYPE_F32, False),
+    # the blocked kernel's two-block form
+    (9, 5, kvc.DTYPE_F32, kvc.DTYPE_F32, True),
+    (12, 8, kvc.DTYPE_F32, kvc.DTYPE_BF16, False),
+    (12, 5, kvc.DTYPE_BF16, kvc.DTYPE_BF16, True),
+    # the one-token kernel's 512-thread form
+    (1, 17, kvc.DTYPE_F32, kvc.DTYPE_F32, False),
+    (1, 17, kvc.DTYPE_F32, kvc.DTYPE_BF16, True),
+    (1, 18, kvc.DTYPE_BF16, kvc.DTYPE_BF16, True),
+])
+def test_many_sequences(n_tok, n_seqs, in_dtype, out_dtype, exact):
+    say(f"deltanet, {n_seqs} sequences of {n_tok} tokens, in {in_dtype} out {out_dtype} exact {exact}")
+    run_case(in_dtype, out_dtype, n_tok=n_tok, n_seqs=n_seqs, seed=12700 + 7 * n_tok + n_seqs, exact=exact)
+
+
+def test_persistent_kernel_long_call_with_almost_no_decay():
+    say("deltanet ranges: 8 sequences of 512 tokens, decays near 1")
+    check_all(*run(512, 8, 13100, a_range=(1e-4, 1e-3)), "512 tokens, weak decay")
 
 
 @pytest.mark.parametrize("case", [

@@ -1,12 +1,13 @@
 """The Gated-DeltaNet matrix form at the edges of its number ranges, against
 the oracle (src/engine.cpp:3197-3327, oracle fast = 1).
 
-The matrix form (calls of 14 or more tokens) computes its state products on
+The matrix form (calls of 13 or more tokens) computes its state products on
 fp16 MFMA: every fp32 operand is split into two fp16 parts after a
 power-of-two scale (one per state column, from a bound carried across the
 blocks), and the blocks' decays accumulate in a per-wave factor that is folded
-back into the state when it falls below 2^-80.  These cases drive each of
-those paths where a wrong scale or a missed fold would show:
+back into the state when it falls below 2^-80.  These cases, with 2 sequences,
+drive each of those paths in the few-sequence launches (test_gpu_deltanet_few.py
+has the persistent kernel's) where a wrong scale or a missed fold would show:
 
 - a long call with almost no decay (32 blocks, the factor never folds, the
   state grows);

@@ -198,7 +198,8 @@ def test_decode_loop_across_blocks(chunk):
 
 
 # Gated-DeltaNet step: token counts across the blocked kernel (2..12, one and
-# two blocks) and the matrix form (13 and more, partial last blocks), with
+# two blocks) and the few-sequence matrix form (13 and more, partial last
+# blocks; more sequences: test_gpu_deltanet_few.py), with
 # every pairing of input and output dtype and both math modes; the state, the
 # conv window and every token's output are checked against the oracle
 # (run_case of test_gpu_deltanet).

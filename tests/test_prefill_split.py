@@ -87,3 +87,10 @@ def test_long_keys_are_cut_within_the_workspace(picks):
                 (3, [100000] * 3)]
     for (n_q, prefix), (rows, piece, slots, most) in zip(launches, picks(launches)):
         assert piece > 0 and slots <= most, (n_q, prefix)
+
+
+def test_routes_of_the_gpu_cases(picks):
+    from test_gpu_prefill_split import CASES
+
+    for case, (rows, piece, _, _) in zip(CASES, picks([(n_q, prefix) for prefix, n_q, _ in CASES])):
+        assert (rows, piece > 0) == case[2], case
