@@ -1,6 +1,6 @@
 """GPU parity of decode's automatic work split at the edges of its rule (one
 chunk per sequence, one workgroup per CU with and without the output-dim
-split, short chunks for very unequal lengths), against the oracle
+split, short chunks where that would leave one long chunk), against the oracle
 (src/engine.cpp:3528-3564): max |diff| <= 2e-2 and relative RMS <= 3e-3; of its
 weight offset under scores that move by hundreds of bits from group to group or
 by one key in any block of a group, with the same bars; and of
@@ -17,14 +17,15 @@ pytestmark = pytest.mark.gpu
 
 CASES = {
     "one_chunk": [1, 31, 96],                 # every sequence in one chunk of 3 blocks
-    "four_blocks": [97],                      # first length in several chunks
+    "four_blocks": [97],                      # first length in several chunks, of one block
     "one_block_chunks": [1024],               # 32 chunks of one block
     "past_32_chunks": [1025],                 # 33 blocks: chunks of two
     "short_launch": [1000, 1024],             # 64 blocks: 32 chunks, two parts
-    "past_short_launch": [1000, 1056],        # 65 blocks: chunks of one block, one part
+    "past_short_launch": [1000, 1056],        # 65 blocks: 33 chunks, one part
     "ragged_one_round": [777, 2001, 65, 1500],
-    "very_ragged": [9000] + [33] * 40,        # short chunks
-    "full_batch": [40 + 7 * i for i in range(64)],
+    "very_ragged": [9000] + [33] * 40,        # 64 chunks of up to 12 blocks
+    "full_batch": [40 + 7 * i for i in range(64)],  # a chunk per sequence
+    "full_batch_ragged": [4000] + [33] * 63,  # short chunks (4 blocks), in rounds
 }
 
 
