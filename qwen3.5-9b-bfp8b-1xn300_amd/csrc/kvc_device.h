@@ -23,12 +23,10 @@ __device__ __forceinline__ uint32_t f32_to_bf16_rne(float x) {
     u += 0x7FFFu + ((u >> 16) & 1u);
     return u >> 16;
 }
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return f32_to_bf16_rne(lo) | (f32_to_bf16_rne(hi) << 16);
-}
 
-// Two finite floats -> packed bf16 pair, round to nearest even, branch free
-// (v_cvt_pk_bf16_f32 on gfx950).  For hot loops whose inputs are never NaN.
+// Two floats -> packed bf16 pair, round to nearest even, branch free
+// (v_cvt_pk_bf16_f32 on gfx950): f32_to_bf16_rne's bits, infinities included;
+// NaN stays a quiet NaN.
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
     const f32x2_t v = {lo, hi};

@@ -28,8 +28,7 @@ __global__ void table_update_kernel(TableUpdateArgs a) {
 // is this lane's share of the softmax denominator for its own head; acc[g][j]
 // holds output dims d = lane*4 + j of q head g of the group.
 struct WaveState {
-    float m[kGroup];  // filled by finalize_l
-    float l[kGroup];
+    float m[kGroup], l[kGroup];  // filled by finalize_l
     // of the lane's head: weight offset (weights are 2^(score - m)), the highest
     // that the offset has been, and the lane's part of the denominator
     float m_lane, top, l_lane;
@@ -51,12 +50,9 @@ struct BlockRegs {
 
 __device__ __forceinline__ void init_state(WaveState& st) {
 #pragma unroll
-    for (int g = 0; g < kGroup; g++) {
-        st.m[g] = kNegBig;
-        st.l[g] = 0.f;
+    for (int g = 0; g < kGroup; g++)
 #pragma unroll
         for (int j = 0; j < 4; j++) st.acc[g][j] = 0.f;
-    }
     st.l_lane = 0.f;
     st.m_lane = st.top = kNegBig;
 }

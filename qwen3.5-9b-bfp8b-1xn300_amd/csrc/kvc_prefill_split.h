@@ -40,10 +40,7 @@ inline void prefill_split(PrefillArgs& a) {
     const auto blocks_of = [&](int rows) { return (a.n_q + rows - 1) / (int64_t)rows; };
     a.rows = 32;
     a.piece_tiles = 0;
-    if (a.n_groups * blocks_of(32) >= 2 * (int64_t)kCus) {
-        if (a.n_q <= 16) a.rows = 16;
-        return;
-    }
+    if (a.n_groups * blocks_of(32) >= 2 * (int64_t)kCus) return;
     double best = 1e30;
     const auto take = [&](double cost, int rows, int64_t piece_tiles) {
         if (cost >= best) return;
