@@ -262,7 +262,9 @@ int kvc_decode_step(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
  * row i attends to keys [0, pos_i].  q/gate: bf16 [n_seqs][n_q][Hq][D];
  * out: [n_seqs][n_q][Hq][D].  A launch too small to fill the GPU splits its
  * keys over workgroups and folds them through the context's split-K
- * workspace. */
+ * workspace.  That split, and with it the rounding (within the bf16 weights'),
+ * follows from the lengths of all seqs of the launch, as decode's does: a row's
+ * bits can differ between calls of different batches. */
 int kvc_prefill_attn(kvc_ctx* ctx, int32_t layer, const int32_t* seqs,
                      int32_t n_seqs, int32_t n_q, const void* q,
                      const void* gate, void* out, int32_t out_dtype,
@@ -327,8 +329,11 @@ int kvc_state_ptrs(kvc_ctx* ctx, int32_t seq, int32_t ssm_layer, void** rec,
  * (each within 2 ulp of the exact function) instead.  Built for
  * 32 v-heads, 16 k-heads, 128 x 128 heads, a 3-row window and 8192 channels
  * (KVC_ERR_UNSUPPORTED otherwise); one seq's n_tok rows of proj must span
- * less than 2 GiB (KVC_ERR_RANGE otherwise).  Calls of few sequences and many
- * tokens run as several launches through the context's split-K workspace. */
+ * less than 2 GiB (KVC_ERR_RANGE otherwise).  Calls of 13 or more tokens
+ * of few sequences run as several launches through the context's split-K
+ * workspace.  Up to 12 tokens a call gives the bits of as many one-token calls;
+ * from 13 the order of its fp32 sums, and with it the last bits, depends on the
+ * number of tokens and seqs of the call. */
 int kvc_deltanet_step(kvc_ctx* ctx, int32_t ssm_layer, const int32_t* seqs,
                       int32_t n_seqs, int32_t n_tok, const void* proj,
                       int32_t in_dtype, const void* conv_w, const void* dt_bias,
