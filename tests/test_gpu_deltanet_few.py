@@ -33,7 +33,7 @@ def test_few_sequences(n_tok, n_seqs, in_dtype, out_dtype):
 
 
 @pytest.mark.parametrize("exact", [False, True])
-@pytest.mark.parametrize("n_seqs", [1, 2, 3, 4])
+@pytest.mark.parametrize("n_seqs", [1, 2, 3, 4, 17])
 @pytest.mark.parametrize("n_tok", [2, 8, 9, 10, 11, 12])
 def test_short_calls_have_the_bits_of_token_steps(n_tok, n_seqs, exact):
     """Up to 12 tokens, however few the sequences, the arithmetic is fp32
@@ -44,7 +44,10 @@ def test_short_calls_have_the_bits_of_token_steps(n_tok, n_seqs, exact):
     OUT = O.SSM_NV * O.SSM_DV
     w = [0.5 * rng.standard_normal((4, O.SSM_C)), rng.standard_normal(O.SSM_NV), -rng.uniform(0.05, 1.0, O.SSM_NV),
          rng.uniform(0.5, 1.5, O.SSM_DV)]
-    proj = O.f32_to_bf16(rng.standard_normal((n_seqs, n_tok, O.SSM_PROJ)).astype(np.float32))
+    proj = rng.standard_normal((n_seqs, n_tok, O.SSM_PROJ)).astype(np.float32)
+    in_dtype = kvc.DTYPE_F32 if n_seqs % 2 else kvc.DTYPE_BF16
+    if in_dtype == kvc.DTYPE_BF16:
+        proj = O.f32_to_bf16(proj)
     S0 = (0.05 * rng.standard_normal(OUT * O.SSM_DK)).astype(np.float32)
     got = []
     with ctx_ssm(max_seqs=2 * n_seqs, flags=kvc.FLAG_EXACT_MATH if exact else 0) as ctx:
@@ -56,7 +59,7 @@ def test_short_calls_have_the_bits_of_token_steps(n_tok, n_seqs, exact):
             out = np.empty((n_seqs, n_tok, OUT), np.float32)
             for t in range(0, n_tok, step):
                 pb, ob = kvc.to_device(np.ascontiguousarray(proj[:, t:t + step])), h.malloc(n_seqs * step * OUT * 4)
-                ctx.deltanet_step(0, seqs, step, pb, *bufs, ob)
+                ctx.deltanet_step(0, seqs, step, pb, *bufs, ob, in_dtype=in_dtype)
                 ctx.sync()
                 out[:, t:t + step] = ob.download(np.float32, (n_seqs, step, OUT))
                 pb.free()
