@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/kvc.h"
+#include "kvc_decode_split.h"
 #include "kvc_internal.h"
 #include "kvc_prefill_split.h"
 
@@ -1086,52 +1087,6 @@ int kvc_qkv_append(kvc_ctx* c, int32_t layer, const int32_t* seqs, int32_t n_seq
         if (e) return hip_err((hipError_t)e, "qkv append launch");
     }
     return KVC_OK;
-}
-
-// Blocks per split-K chunk when the caller leaves it open, from the sequences'
-// block counts nb[n].  Two ways to cut a launch:
-//  - one workgroup per CU (at most 64 chunks x 4 heads, 32 chunks per
-//    sequence for a short combine): the CUs share HBM, so it takes the time of
-//    its bytes plus what the longest chunk has over the mean, at 0.45 us per
-//    block of a workgroup alone;
-//  - short chunks in many rounds, which balance ragged sequences: an item costs
-//    7 ns of the launch's time, the last one of a CU 0.45 us per block, least
-//    at 0.25 sqrt(total blocks) per chunk.
-// The cheaper by that estimate is taken.  us per layer of kvc_decode_step, the
-// former rule (4-block chunks, more only past 4096 items) -> this one: 1
-// sequence of 300 tokens 7.74 -> 6.51, 2000 8.11 -> 7.39, 4200 10.35 -> 9.21,
-// 32768 38.0 -> 27.3; 64 of 300 27.9 -> 19.0; 64 of 1000 59.6 -> 45.5; 8 of
-// 777-6001 33.0 -> 26.3; kvc_decode_attn of 64 of 512-32768 (short chunks,
-// fewer than before) 723 -> 703.
-static int32_t auto_chunk_blocks(const int32_t* nb, int32_t n, bool force_split) {
-    int64_t total = 0;
-    int32_t longest = 1;
-    for (int32_t j = 0; j < n; j++) {
-        total += nb[j];
-        longest = std::max(longest, nb[j]);
-    }
-    // a chunk per sequence needs no exchange: 64 tokens 5.6 us, in two chunks 6.4
-    if (longest <= 3) return 3;
-    // short launches do better with two output-dim parts per chunk than with
-    // twice the chunks: 2 sequences of 1000 tokens 7.6 us against 8.3
-    const int32_t max_chunks = force_split || total <= 64 ? 32 : 64;
-    const auto chunks = [&](int32_t cb) {
-        int64_t c = 0;
-        for (int32_t j = 0; j < n; j++) c += (nb[j] + cb - 1) / cb;
-        return c;
-    };
-    const int32_t short_cb = std::max(4, (int32_t)std::lround(0.25 * std::sqrt((double)total)));
-    if (n > max_chunks) return total <= 64 ? 3 : short_cb;
-    // smallest cb with at most max_chunks chunks (monotone in cb)
-    int32_t lo = std::max<int32_t>((longest + 31) / 32, (int32_t)((total + max_chunks - 1) / max_chunks)), hi = longest;
-    while (lo < hi) {
-        const int32_t mid = (lo + hi) / 2;
-        if (chunks(mid) <= max_chunks)
-            hi = mid;
-        else
-            lo = mid + 1;
-    }
-    return lo - total / 64.0 <= 0.5 * std::sqrt((double)total) ? lo : short_cb;
 }
 
 // Argument block of the decode launch over seqs[i0, i0 + n): work split and

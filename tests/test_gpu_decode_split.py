@@ -21,7 +21,9 @@ CASES = {
     "one_block_chunks": [1024],               # 32 chunks of one block
     "past_32_chunks": [1025],                 # 33 blocks: chunks of two
     "short_launch": [1000, 1024],             # 64 blocks: 32 chunks, two parts
-    "past_short_launch": [1000, 1056],        # 65 blocks: 33 chunks, one part
+    "four_blocks_many": [97 + 2 * i for i in range(13)],  # a chunk per sequence again
+    "past_short_launch": [1000, 1056],        # 65 blocks: 22 chunks, two parts
+    "past_short_launch_one_part": [700] * 3,  # 66 blocks: 33 chunks, one part
     "ragged_one_round": [777, 2001, 65, 1500],
     "very_ragged": [9000] + [33] * 40,        # 64 chunks of up to 12 blocks
     "full_batch": [40 + 7 * i for i in range(64)],  # a chunk per sequence
